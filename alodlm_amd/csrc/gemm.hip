@@ -13,6 +13,7 @@
 // float path and unaligned shapes: a plain LDS-tiled FMA kernel.
 #include "common.h"
 #include "gemm_dl.h"
+#include "gemm_skinny.h"
 
 typedef __attribute__((__vector_size__(8 * sizeof(short)))) short bf16x8_t;
 typedef __attribute__((__vector_size__(16 * sizeof(float)))) float f32x16_t;
@@ -431,6 +432,12 @@ extern "C" int alodlm_gemm(const void* A, int64_t lda, int a_kmajor, const void*
   ALODLM_CHECK_ARG(epilogue != ALODLM_EPI_RESIDUAL || R != nullptr, "gemm: residual needs R");
   if (M == 0 || N == 0) return ALODLM_OK;
   hipStream_t st = as_stream(stream);
+  if ((dtype == ALODLM_BF16 || dtype == ALODLM_F32) &&
+      gemm_skinny_eligible(A, lda, a_kmajor, B, ldb, b_kmajor, M, N, K, epilogue, dtype)) {
+    gemm_skinny_launch(A, lda, B, ldb, C, ldc, R, ldr, M, N, K, alpha, epilogue, dtype, st);
+    ALODLM_CHECK_LAUNCH("gemm_skinny");
+    return ALODLM_OK;
+  }
   if (dtype == ALODLM_BF16 && mfma_eligible(A, lda, a_kmajor, B, ldb, b_kmajor, M, N, K) &&
       gemm_dl_eligible(lda, a_kmajor, ldb, b_kmajor, M, N, K)) {
     int64_t splits = 1;

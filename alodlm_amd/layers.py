@@ -31,6 +31,7 @@ from . import _lib
 from ._lib import EPI_ACCUM, EPI_RESIDUAL, EPI_STORE, EPI_STORE_F32, call, ptr, query
 
 TILE_ROWS = 128
+SKINNY_ROWS = 64  # rows up to which a product streams its [out, in] weight
 
 
 def allowed_pairs(length, block_size):
@@ -330,8 +331,9 @@ class Kernels:
 
     def _product(self, x, ldx, w, w_t, y, M, N, K, epi=EPI_STORE, R=None, ldr=0):
         """y = x . w^T (+ R) with w [N, K]: through the out-contiguous copy w_t
-        [K, N] when there is one."""
-        if w_t is not None:
+        [K, N] when there is one and M rows fill the wide tiles it serves
+        (fewer rows stream w itself, whose rows are k-contiguous)."""
+        if w_t is not None and M > SKINNY_ROWS:
             self._gemm(x, ldx, 1, w_t, N, 0, y, N, M, N, K, epi=epi, R=R, ldr=ldr)
         else:
             self._gemm(x, ldx, 1, w, K, 1, y, N, M, N, K, epi=epi, R=R, ldr=ldr)
