@@ -10,9 +10,13 @@
 // loads and writes four 16-byte k-rows.  Global loads for tile k+1 are issued
 // before the MFMAs of tile k (register prefetch, double-buffered LDS).
 //
-// float path and unaligned shapes: a plain LDS-tiled FMA kernel.
+// float: gemm_f32.hip; few rows: gemm_skinny.hip; unaligned shapes: a plain
+// LDS-tiled FMA kernel.
+#include <type_traits>
+
 #include "common.h"
 #include "gemm_dl.h"
+#include "gemm_f32.h"
 #include "gemm_skinny.h"
 
 typedef __attribute__((__vector_size__(8 * sizeof(short)))) short bf16x8_t;
@@ -210,77 +214,78 @@ gemm_bf16_kernel(const bf16_t* __restrict__ A, int64_t lda, const bf16_t* __rest
     }
 }
 
-// C[m, n] (+)= sum_s partial[s, m, n] (partials summed in split order, then
-// added to C, or written over it when `overwrite`)
+// The epilogue of a split product from its float partials (which carry alpha),
+// summed in split order: STORE C = s, RESIDUAL C = R + cast(s), ACCUM C += s
+// (float C), each rounded once.  VEC columns per thread (4: N, ldc, ldr
+// multiples of 4 and every row of the buffers aligned to 4 elements); grid.x
+// covers a row's column groups and grid.y strides over rows, so no 64-bit
+// division is needed.
+template <typename T, int EPI, int VEC>
 __global__ void splitk_reduce_kernel(const float* __restrict__ partial, int64_t splits, int64_t M,
-                                     int64_t N, float* __restrict__ C, int64_t ldc,
-                                     bool overwrite) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= M * N) return;
-  float s = 0.f;
-  for (int64_t p = 0; p < splits; ++p) s += partial[p * M * N + i];
-  float* dst = C + (i / N) * ldc + (i % N);
-  *dst = overwrite ? s : *dst + s;
-}
-
-// The same sum, 4 consecutive columns per thread (N, ldc multiples of 4, both
-// buffers 16-byte aligned): grid.x covers a row's N/4 column groups, grid.y
-// strides over rows, so no 64-bit division is needed.
-__global__ void splitk_reduce4_kernel(const float* __restrict__ partial, int64_t splits,
-                                      int64_t M, int64_t N, float* __restrict__ C, int64_t ldc,
-                                      bool overwrite) {
-  const int64_t n = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * 4;
+                                     int64_t N, T* C, int64_t ldc, const T* R, int64_t ldr) {
+  const int64_t n = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * VEC;
   if (n >= N) return;
   const int64_t plane = M * N;
   for (int64_t m = blockIdx.y; m < M; m += gridDim.y) {
     const float* src = partial + m * N + n;
-    float4 s = *reinterpret_cast<const float4*>(src);
-    for (int64_t p = 1; p < splits; ++p) {
-      const float4 t = *reinterpret_cast<const float4*>(src + p * plane);
-      s.x += t.x; s.y += t.y; s.z += t.z; s.w += t.w;
-    }
-    float4* dst = reinterpret_cast<float4*>(C + m * ldc + n);
-    if (overwrite) {
-      *dst = s;
+    float s[VEC];
+    if constexpr (VEC == 4) {
+      float4 t = *reinterpret_cast<const float4*>(src);
+      for (int64_t p = 1; p < splits; ++p) {
+        const float4 u = *reinterpret_cast<const float4*>(src + p * plane);
+        t.x += u.x; t.y += u.y; t.z += u.z; t.w += u.w;
+      }
+      s[0] = t.x; s[1] = t.y; s[2] = t.z; s[3] = t.w;
     } else {
-      float4 c = *dst;
-      c.x += s.x; c.y += s.y; c.z += s.z; c.w += s.w;
-      *dst = c;
+      s[0] = src[0];
+      for (int64_t p = 1; p < splits; ++p) s[0] += src[p * plane];
+    }
+    T* dst = C + m * ldc + n;
+    if constexpr (EPI == ALODLM_EPI_RESIDUAL || EPI == ALODLM_EPI_ACCUM) {
+      T r[VEC];
+      __builtin_memcpy(r, EPI == ALODLM_EPI_RESIDUAL ? R + m * ldr + n : dst, sizeof(r));
+#pragma unroll
+      for (int e = 0; e < VEC; ++e) s[e] = Elem<T>::load(r, e) + Elem<T>::round(s[e]);
+    }
+    if constexpr (VEC == 4 && std::is_same<T, bf16_t>::value) {
+      *reinterpret_cast<uint2*>(dst) = make_uint2(pack_bf16x2(s[0], s[1]), pack_bf16x2(s[2], s[3]));
+    } else if constexpr (VEC == 4) {
+      *reinterpret_cast<float4*>(dst) = make_float4(s[0], s[1], s[2], s[3]);
+    } else {
+      Elem<T>::store(dst, 0, s[0]);
     }
   }
 }
 
-// C[m, n] = bf16(sum_s partial[s, m, n]) (split order; the partials carry
-// alpha): the STORE epilogue of a split product, rounded once.
-__global__ void splitk_store_kernel(const float* __restrict__ partial, int64_t splits, int64_t M,
-                                    int64_t N, bf16_t* __restrict__ C, int64_t ldc) {
-  const int64_t n = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (n >= N) return;
-  const int64_t plane = M * N;
-  for (int64_t m = blockIdx.y; m < M; m += gridDim.y) {
-    float s = partial[m * N + n];
-    for (int64_t p = 1; p < splits; ++p) s += partial[p * plane + m * N + n];
-    C[m * ldc + n] = float_to_bf16(s);
-  }
+template <typename T, int EPI>
+static void splitk_launch(const float* partial, int64_t splits, int64_t M, int64_t N, T* C,
+                          int64_t ldc, const T* R, int64_t ldr, hipStream_t st) {
+  const bool residual = EPI == ALODLM_EPI_RESIDUAL;
+  const bool vec = N % 4 == 0 && ldc % 4 == 0 && (!residual || ldr % 4 == 0) &&
+                   reinterpret_cast<uintptr_t>(partial) % 16 == 0 &&
+                   reinterpret_cast<uintptr_t>(C) % (4 * sizeof(T)) == 0 &&
+                   (!residual || reinterpret_cast<uintptr_t>(R) % (4 * sizeof(T)) == 0);
+  const dim3 grid(ceil_div_u(vec ? N / 4 : N, 256), (unsigned)(M < 65535 ? M : 65535));
+  if (vec) splitk_reduce_kernel<T, EPI, 4><<<grid, 256, 0, st>>>(partial, splits, M, N, C, ldc, R, ldr);
+  else splitk_reduce_kernel<T, EPI, 1><<<grid, 256, 0, st>>>(partial, splits, M, N, C, ldc, R, ldr);
 }
 
-static void splitk_store(const float* partial, int64_t splits, int64_t M, int64_t N, bf16_t* C,
-                         int64_t ldc, hipStream_t st) {
-  const dim3 grid(ceil_div_u(N, 256), (unsigned)(M < 65535 ? M : 65535));
-  splitk_store_kernel<<<grid, 256, 0, st>>>(partial, splits, M, N, C, ldc);
-}
-
-static void splitk_reduce(const float* partial, int64_t splits, int64_t M, int64_t N, float* C,
-                          int64_t ldc, hipStream_t st, bool overwrite = false) {
-  const bool vec = N % 4 == 0 && ldc % 4 == 0 &&
-                   ((reinterpret_cast<uintptr_t>(partial) | reinterpret_cast<uintptr_t>(C)) & 15) == 0;
-  if (vec) {
-    const dim3 grid(ceil_div_u(N / 4, 256), (unsigned)(M < 65535 ? M : 65535));
-    splitk_reduce4_kernel<<<grid, 256, 0, st>>>(partial, splits, M, N, C, ldc, overwrite);
-  } else {
-    splitk_reduce_kernel<<<ceil_div_u(M * N, 256), 256, 0, st>>>(partial, splits, M, N, C, ldc,
-                                                                 overwrite);
-  }
+// C in `dtype` for STORE / RESIDUAL, float for ACCUM / STORE_F32.
+static void splitk_reduce(const float* partial, int64_t splits, int64_t M, int64_t N, void* C,
+                          int64_t ldc, const void* R, int64_t ldr, int epi, int dtype,
+                          hipStream_t st) {
+  if (epi == ALODLM_EPI_ACCUM)
+    splitk_launch<float, ALODLM_EPI_ACCUM>(partial, splits, M, N, (float*)C, ldc, nullptr, 0, st);
+  else if (epi == ALODLM_EPI_STORE_F32 || (epi == ALODLM_EPI_STORE && dtype == ALODLM_F32))
+    splitk_launch<float, ALODLM_EPI_STORE>(partial, splits, M, N, (float*)C, ldc, nullptr, 0, st);
+  else if (epi == ALODLM_EPI_STORE)
+    splitk_launch<bf16_t, ALODLM_EPI_STORE>(partial, splits, M, N, (bf16_t*)C, ldc, nullptr, 0, st);
+  else if (dtype == ALODLM_F32)
+    splitk_launch<float, ALODLM_EPI_RESIDUAL>(partial, splits, M, N, (float*)C, ldc,
+                                              (const float*)R, ldr, st);
+  else
+    splitk_launch<bf16_t, ALODLM_EPI_RESIDUAL>(partial, splits, M, N, (bf16_t*)C, ldc,
+                                               (const bf16_t*)R, ldr, st);
 }
 
 // C[m, n] = 0 for an [M, N] float matrix with row stride ldc (a fill kernel,
@@ -297,7 +302,7 @@ static void zero_rows(float* C, int64_t M, int64_t N, int64_t ldc, hipStream_t s
 }
 
 // ---------------------------------------------------------------------------
-// Generic LDS-tiled FMA kernel (float, or any layout/shape).  64x64 tile,
+// Generic LDS-tiled FMA kernel (any layout, shape and alignment).  64x64 tile,
 // 256 threads with 4x4 outputs each, k-step 16.
 // ---------------------------------------------------------------------------
 template <typename T, int EPI>
@@ -383,7 +388,10 @@ static bool use_big(int64_t M, int64_t N, int64_t K, bool any_kmajor = false) {
 }
 
 extern "C" int64_t alodlm_gemm_workspace(int64_t M, int64_t N, int64_t K, int epilogue, int dtype) {
-  if (dtype != ALODLM_BF16) return 0;
+  if (dtype != ALODLM_BF16) {
+    const int64_t s = dtype == ALODLM_F32 && M > 0 && N > 0 ? gemm_f32_splits(M, N, K) : 1;
+    return s > 1 ? s * M * N : 0;
+  }
   if (epilogue == ALODLM_EPI_STORE) {
     const int64_t s = (M >= 256 && N >= 256 && K % 32 == 0) ? gemm_dl_store_splits(M, N, K) : 1;
     return s > 1 ? s * M * N : 0;
@@ -420,7 +428,7 @@ static void launch_mfma(const bf16_t* A, int64_t lda, const bf16_t* B, int64_t l
   else
     gemm_bf16_kernel<AK, BK, ALODLM_EPI_ACCUM><<<grid, GM_THREADS, 0, st>>>(
         A, lda, B, ldb, C, ldc, R, ldr, M, N, K, alpha, kps, part);
-  if (part) splitk_reduce(part, nsplit, M, N, (float*)C, ldc, st);
+  if (part) splitk_reduce(part, nsplit, M, N, C, ldc, nullptr, 0, epi, ALODLM_BF16, st);
 }
 
 extern "C" int alodlm_gemm(const void* A, int64_t lda, int a_kmajor, const void* B, int64_t ldb,
@@ -461,10 +469,21 @@ extern "C" int alodlm_gemm(const void* A, int64_t lda, int a_kmajor, const void*
                    first_into_c, st);
     ALODLM_CHECK_LAUNCH("gemm_bf16_dl");
     if ((launch_epi == ALODLM_EPI_ACCUM || launch_epi == ALODLM_EPI_STORE_F32) && nsplit > 1) {
-      if (epilogue == ALODLM_EPI_STORE) splitk_store(workspace, nsplit, M, N, (bf16_t*)C, ldc, st);
-      else if (first_into_c) splitk_reduce(workspace + M * N, nsplit - 1, M, N, (float*)C, ldc, st);
-      else splitk_reduce(workspace, nsplit, M, N, (float*)C, ldc, st,
-                         epilogue == ALODLM_EPI_STORE_F32);
+      if (first_into_c)
+        splitk_reduce(workspace + M * N, nsplit - 1, M, N, C, ldc, nullptr, 0, epilogue, dtype, st);
+      else
+        splitk_reduce(workspace, nsplit, M, N, C, ldc, nullptr, 0, epilogue, dtype, st);
+      ALODLM_CHECK_LAUNCH("gemm_splitk_reduce");
+    }
+    return ALODLM_OK;
+  }
+  if (dtype == ALODLM_F32 && gemm_f32_eligible(A, lda, a_kmajor, B, ldb, b_kmajor, M, N, K)) {
+    const int64_t nsplit = gemm_f32_launch((const float*)A, lda, a_kmajor, (const float*)B, ldb,
+                                           b_kmajor, (float*)C, ldc, (const float*)R, ldr, M, N, K,
+                                           alpha, epilogue, workspace, st);
+    ALODLM_CHECK_LAUNCH("gemm_f32");
+    if (nsplit > 1) {
+      splitk_reduce(workspace, nsplit, M, N, C, ldc, R, ldr, epilogue, dtype, st);
       ALODLM_CHECK_LAUNCH("gemm_splitk_reduce");
     }
     return ALODLM_OK;
@@ -487,7 +506,7 @@ extern "C" int alodlm_gemm(const void* A, int64_t lda, int a_kmajor, const void*
                     (const bf16_t*)R, ldr, M, N, K, alpha, epilogue, workspace, splits, &nsplit, st);
     ALODLM_CHECK_LAUNCH("gemm_bf16_256");
     if (epilogue == ALODLM_EPI_ACCUM && nsplit > 1) {
-      splitk_reduce(workspace, nsplit, M, N, (float*)C, ldc, st);
+      splitk_reduce(workspace, nsplit, M, N, C, ldc, nullptr, 0, epilogue, dtype, st);
       ALODLM_CHECK_LAUNCH("gemm_splitk_reduce");
     }
     return ALODLM_OK;
@@ -562,8 +581,8 @@ extern "C" int alodlm_gemm_segk(const void* const* a_segs, const void* const* b_
                  epilogue, workspace, splits, &nsplit, first_into_c, st, &segs);
   ALODLM_CHECK_LAUNCH("gemm_bf16_dl_segk");
   if (nsplit > 1) {
-    if (first_into_c) splitk_reduce(workspace + M * N, nsplit - 1, M, N, (float*)C, ldc, st);
-    else splitk_reduce(workspace, nsplit, M, N, (float*)C, ldc, st, true);
+    splitk_reduce(first_into_c ? workspace + M * N : workspace, nsplit - first_into_c, M, N, C, ldc,
+                  nullptr, 0, epilogue, ALODLM_BF16, st);
     ALODLM_CHECK_LAUNCH("gemm_splitk_reduce");
   }
   return ALODLM_OK;

@@ -192,9 +192,8 @@ int alodlm_rotary_bwd(const void* dout, const void* cos_tab, const void* sin_tab
  *           ALODLM_EPI_STORE_F32 Cf32 = alpha*acc            (C is float: the first
  *                               contribution to a gradient, which then needs no zeroing)
  * workspace: float scratch of alodlm_gemm_workspace(M, N, K, epilogue, dtype)
- * floats for split-K partials: ALODLM_EPI_ACCUM products with few output
- * tiles, and bf16 ALODLM_EPI_STORE products with K >= 16384 and few output
- * tiles (summed in split order, then rounded once).  May be NULL (the
+ * floats for split-K partials of products with few output tiles (summed in
+ * split order, then rounded once).  May be NULL (the
  * product then runs unsplit); unused when the query returns 0.
  * ------------------------------------------------------------------------ */
 enum { ALODLM_EPI_STORE = 0, ALODLM_EPI_RESIDUAL = 1, ALODLM_EPI_ACCUM = 2,
