@@ -6,58 +6,16 @@
 // rows of its own block.  The kernels enumerate exactly those key ranges, so
 // no masked pair and no cross-segment pair is ever visited.
 //
+// bf16 with head_dim 64 or 128 runs attention_mfma.hip / attention_fa128.hip,
+// float with head_dim 128 attention_f32.hip.
 // Reference kernels (any dtype, any head_dim): one wavefront per (query row,
 // head) in the forward and dQ passes and one per (key row, kv head) in the
 // dK/dV pass; the wavefront spreads head_dim over its lanes.
 #include <initializer_list>
 
-#include "common.h"
+#include "attention_common.h"
 
 #define ATT_MAX_PER_LANE 4  // head_dim <= 256
-
-struct SegRow {
-  int64_t base, L, i;  // segment start row, segment length, in-segment index (0..2L)
-};
-
-__device__ __forceinline__ SegRow seg_row(const int64_t* bounds, const int32_t* row_segment,
-                                          int64_t r) {
-  const int32_t s = row_segment[r];
-  SegRow o;
-  o.base = bounds[s];
-  o.L = (bounds[s + 1] - o.base) / 2;
-  o.i = r - o.base;
-  return o;
-}
-
-// Key ranges [k0a, k1a) and [k0b, k1b) (absolute rows) seen by query row r.
-__device__ __forceinline__ void query_key_ranges(const SegRow& q, int64_t B, int64_t& k0a,
-                                                 int64_t& k1a, int64_t& k0b, int64_t& k1b) {
-  if (q.i < q.L) {  // clean: causal over the clean stream
-    k0a = q.base; k1a = q.base + q.i + 1;
-    k0b = k1b = 0;
-  } else {
-    const int64_t j = q.i - q.L, blk = j / B;
-    const int64_t clean_end = blk * B < q.L ? blk * B : q.L;
-    k0a = q.base; k1a = q.base + clean_end;
-    k0b = q.base + q.L + blk * B; k1b = q.base + q.i + 1;
-  }
-}
-
-// Query ranges [q0a, q1a) and [q0b, q1b) (absolute rows) that see key row r.
-__device__ __forceinline__ void key_query_ranges(const SegRow& k, int64_t B, int64_t& q0a,
-                                                 int64_t& q1a, int64_t& q0b, int64_t& q1b) {
-  if (k.i < k.L) {
-    const int64_t blk = k.i / B;
-    q0a = k.base + k.i; q1a = k.base + k.L;                  // later clean rows
-    const int64_t first = (blk + 1) * B;                      // noisy rows of later blocks
-    q0b = k.base + k.L + (first < k.L ? first : k.L); q1b = k.base + 2 * k.L;
-  } else {
-    const int64_t j = k.i - k.L, blk = j / B;
-    const int64_t end = (blk + 1) * B < k.L ? (blk + 1) * B : k.L;
-    q0a = k.base + k.i; q1a = k.base + k.L + end;             // same noisy block, causal
-    q0b = q1b = 0;
-  }
-}
 
 template <typename T>
 __global__ void __launch_bounds__(256)
@@ -257,6 +215,26 @@ int fa128_bwd_launch(const bf16_t* q, const bf16_t* k, const bf16_t* v, int64_t 
                      bf16_t* dk, bf16_t* dv, int64_t lddv, int64_t N, int nq, int nkv, int B,
                      float scale, const int64_t* ds_base, int64_t ds_blocks, hipStream_t st);
 
+bool attn_f32_eligible(int64_t rows, int64_t nq, int64_t nkv, int64_t dh, int64_t ldv);
+void attn_f32_fwd_launch(const float* q, const float* k, const float* v, int64_t ldv,
+                         const int64_t* bounds, const int32_t* row_segment, float* o, float* lse,
+                         int64_t rows, int64_t nq, int64_t nkv, int64_t B, float scale,
+                         hipStream_t st);
+void attn_f32_bwd_launch(const float* q, const float* k, const float* v, int64_t ldv,
+                         const float* lse, const float* delta, const float* dout,
+                         const int64_t* bounds, const int32_t* row_segment, float* dq, float* dk,
+                         float* dv, int64_t lddv, int64_t rows, int64_t nq, int64_t nkv, int64_t B,
+                         float scale, hipStream_t st);
+
+// The float matrix-core kernels take head_dim 128 and 16-byte aligned rows.
+static bool use_f32(int dtype, int64_t rows, int64_t nq, int64_t nkv, int64_t dh, int64_t ldv,
+                    std::initializer_list<const void*> ptrs) {
+  if (dtype != ALODLM_F32 || !attn_f32_eligible(rows, nq, nkv, dh, ldv)) return false;
+  for (const void* p : ptrs)
+    if (reinterpret_cast<uintptr_t>(p) % 16) return false;
+  return true;
+}
+
 // The MFMA kernels take bf16, head_dim 64 or 128, 16-byte aligned rows and a
 // tile table; everything else runs the reference kernels above.
 static bool use_mfma(int dtype, int64_t dh, const int32_t* tiles, int64_t ldv,
@@ -286,6 +264,13 @@ extern "C" int alodlm_attention_fwd(const void* q, const void* k, const void* v,
     return fa_fwd_launch((const bf16_t*)q, (const bf16_t*)k, (const bf16_t*)v, ldv, bounds, tiles,
                          n_tiles, (bf16_t*)o, lse, rows, (int)nq, (int)nkv, (int)dh,
                          (int)block_size, scale, as_stream(stream));
+  }
+  if (use_f32(dtype, rows, nq, nkv, dh, ldv, {q, k, v, o})) {
+    attn_f32_fwd_launch((const float*)q, (const float*)k, (const float*)v, ldv, bounds,
+                        row_segment, (float*)o, lse, rows, nq, nkv, block_size, scale,
+                        as_stream(stream));
+    ALODLM_CHECK_LAUNCH("attention_fwd_f32");
+    return ALODLM_OK;
   }
   ALODLM_DISPATCH(dtype, T, {
     attn_fwd_ref_kernel<T><<<ceil_div_u(rows * nq, 4), 256, 0, as_stream(stream)>>>(
@@ -361,6 +346,13 @@ extern "C" int alodlm_attention_bwd(const void* q, const void* k, const void* v,
                          (const bf16_t*)dout, bounds, tiles, n_tiles, (bf16_t*)dq, (bf16_t*)dk,
                          (bf16_t*)dv, lddv, rows, (int)nq, (int)nkv, (int)dh, (int)block_size,
                          scale, st);
+  }
+  if (use_f32(dtype, rows, nq, nkv, dh, ldv, {q, k, v, dout, dq, dk, dv}) && lddv % 4 == 0) {
+    attn_f32_bwd_launch((const float*)q, (const float*)k, (const float*)v, ldv, lse, delta,
+                        (const float*)dout, bounds, row_segment, (float*)dq, (float*)dk,
+                        (float*)dv, lddv, rows, nq, nkv, block_size, scale, st);
+    ALODLM_CHECK_LAUNCH("attention_bwd_f32");
+    return ALODLM_OK;
   }
   ALODLM_DISPATCH(dtype, T, {
     attn_dq_ref_kernel<T><<<ceil_div_u(rows * nq, 4), 256, 0, st>>>(

@@ -115,3 +115,49 @@ __device__ __forceinline__ bool range_next(const Interval2& R, int step, int& r,
   pos = R.lo1;
   return pos < R.hi1;
 }
+
+// The same intervals for one row of the pack, from the row's segment (kernels
+// that take any rows instead of 128-row tiles).
+struct SegRow {
+  int64_t base, L, i;  // segment start row, segment length, in-segment index (0..2L)
+};
+
+__device__ __forceinline__ SegRow seg_row(const int64_t* bounds, const int32_t* row_segment,
+                                          int64_t r) {
+  const int32_t s = row_segment[r];
+  SegRow o;
+  o.base = bounds[s];
+  o.L = (bounds[s + 1] - o.base) / 2;
+  o.i = r - o.base;
+  return o;
+}
+
+// Key ranges [k0a, k1a) and [k0b, k1b) (absolute rows) seen by query row r.
+__device__ __forceinline__ void query_key_ranges(const SegRow& q, int64_t B, int64_t& k0a,
+                                                 int64_t& k1a, int64_t& k0b, int64_t& k1b) {
+  if (q.i < q.L) {  // clean: causal over the clean stream
+    k0a = q.base; k1a = q.base + q.i + 1;
+    k0b = k1b = 0;
+  } else {
+    const int64_t j = q.i - q.L, blk = j / B;
+    const int64_t clean_end = blk * B < q.L ? blk * B : q.L;
+    k0a = q.base; k1a = q.base + clean_end;
+    k0b = q.base + q.L + blk * B; k1b = q.base + q.i + 1;
+  }
+}
+
+// Query ranges [q0a, q1a) and [q0b, q1b) (absolute rows) that see key row r.
+__device__ __forceinline__ void key_query_ranges(const SegRow& k, int64_t B, int64_t& q0a,
+                                                 int64_t& q1a, int64_t& q0b, int64_t& q1b) {
+  if (k.i < k.L) {
+    const int64_t blk = k.i / B;
+    q0a = k.base + k.i; q1a = k.base + k.L;                  // later clean rows
+    const int64_t first = (blk + 1) * B;                      // noisy rows of later blocks
+    q0b = k.base + k.L + (first < k.L ? first : k.L); q1b = k.base + 2 * k.L;
+  } else {
+    const int64_t j = k.i - k.L, blk = j / B;
+    const int64_t end = (blk + 1) * B < k.L ? (blk + 1) * B : k.L;
+    q0a = k.base + k.i; q1a = k.base + k.L + end;             // same noisy block, causal
+    q0b = q1b = 0;
+  }
+}
