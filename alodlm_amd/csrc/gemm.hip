@@ -17,6 +17,7 @@
 #include "common.h"
 #include "gemm_dl.h"
 #include "gemm_f32.h"
+#include "gemm_mid.h"
 #include "gemm_skinny.h"
 
 typedef __attribute__((__vector_size__(8 * sizeof(short)))) short bf16x8_t;
@@ -387,23 +388,82 @@ static bool use_big(int64_t M, int64_t N, int64_t K, bool any_kmajor = false) {
   return M >= 256 && N >= 256 && K >= 64 && (!any_kmajor || K % 64 == 0);
 }
 
+// Which kernel a bf16 product runs on and how often its K is split: the one
+// with the least modelled time, from what both measured on the chip.
+//  * 256x256 tiles (gemm_dl.hip): a 32-deep step of a round of 256 workgroups
+//    takes 0.58 us on an idle chip and 0.78 us on a full one (power);
+//  * 128x128 tiles (gemm_mid.hip): 0.28 us (L2 to LDS), for a quarter of the
+//    work; 32 or 64 rows: 0.3 us (the weights' bytes from memory);
+//  * a split's partial sums: written and read at 5.5 TB/s and one launch.
+// Measured against the model's choice at 777 rows (2048 x 6144): 37 us on 128
+// tiles, K in 2, against 113 on 256 tiles; 2474 rows, 12288 x 2048: 102 us on
+// 256 tiles against 169.  The long-K and weight-gradient splits of the 256
+// tiles stay as gemm_dl.hip has them.
+struct Bf16Plan {
+  bool mid;
+  int64_t splits;
+  double cost;
+};
+static Bf16Plan bf16_plan(int64_t M, int64_t N, int64_t K, int epi, int a_kmajor, bool dl_ok,
+                          bool mid_ok, bool workspace) {
+  const bool f32_out = epi == ALODLM_EPI_ACCUM || epi == ALODLM_EPI_STORE_F32;
+  const int64_t cus = 256, steps = (K + 31) / 32;
+  auto reduce = [&](int64_t s) {
+    return s > 1 ? 4.0 + 1e-6 / 5.5 * 4.0 * (double)(2 * s + 1) * (double)M * (double)N : 0.0;
+  };
+  auto cost = [&](int64_t tiles, int64_t s, bool mid, double step) {
+    const double fill = tiles * s < cus ? (double)(tiles * s) / (double)cus : 1.0;
+    const double each = mid ? step : 0.58 + 0.2 * fill;
+    return (double)((tiles * s + cus - 1) / cus) * (double)((steps + s - 1) / s) * each + reduce(s);
+  };
+  Bf16Plan best{false, 1, 1e30};
+  auto offer = [&](bool mid, int64_t s, double c) {
+    if (c < best.cost) best = Bf16Plan{mid, s, c};
+  };
+  if (dl_ok) {
+    const int64_t tiles = ((M + 255) / 256) * ((N + 255) / 256);
+    if (!workspace) offer(false, 1, cost(tiles, 1, false, 0));
+    else if (f32_out || (epi == ALODLM_EPI_STORE && K >= 16384)) {
+      const int64_t s = f32_out ? gemm_dl_splits(M, N, K) : gemm_dl_store_splits(M, N, K);
+      offer(false, s, cost(tiles, s, false, 0));
+    } else {
+      for (int64_t s = 1; s <= 8 && (s == 1 || steps / s >= 16); ++s)
+        offer(false, s, cost(tiles, s, false, 0));
+    }
+  }
+  // float outputs of the 256 tiles keep their kernel and splits: a product over
+  // segments (alodlm_gemm_segk) gives the same bits as one over their
+  // concatenation
+  if (mid_ok && !(f32_out && dl_ok)) {
+    const int rows = gemm_mid_rows(a_kmajor, M, epi);
+    const int64_t tiles = ((M + rows - 1) / rows) * ((N + 127) / 128);
+    const double step = rows == 128 ? 0.28 : 0.3;
+    for (int64_t s = 1; s <= 16 && (s == 1 || (workspace && steps / s >= 8)); ++s)
+      offer(true, s, cost(tiles, s, true, step));
+  }
+  return best;
+}
+
 extern "C" int64_t alodlm_gemm_workspace(int64_t M, int64_t N, int64_t K, int epilogue, int dtype) {
   if (dtype != ALODLM_BF16) {
     const int64_t s = dtype == ALODLM_F32 && M > 0 && N > 0 ? gemm_f32_splits(M, N, K) : 1;
     return s > 1 ? s * M * N : 0;
   }
-  if (epilogue == ALODLM_EPI_STORE) {
-    const int64_t s = (M >= 256 && N >= 256 && K % 32 == 0) ? gemm_dl_store_splits(M, N, K) : 1;
-    return s > 1 ? s * M * N : 0;
+  // the largest of what the product may be given (its layouts and alignment
+  // are not known here)
+  int64_t s = 1;
+  const bool dl_ok = M >= 256 && N >= 256 && K >= 32 && K % 32 == 0;
+  for (int flags = 0; flags < 4; ++flags) {
+    const bool mid_ok = flags & 1;
+    if (!mid_ok && !dl_ok) continue;
+    const Bf16Plan p = bf16_plan(M, N, K, epilogue, flags >> 1, dl_ok, mid_ok, true);
+    s = p.splits > s ? p.splits : s;
   }
-  if (epilogue != ALODLM_EPI_ACCUM && epilogue != ALODLM_EPI_STORE_F32) return 0;
-  int64_t s = splitk_count(M, N, K);
-  if (use_big(M, N, K)) {
-    const int64_t b = gemm_big_splits(M, N, K);
+  if (epilogue == ALODLM_EPI_ACCUM || epilogue == ALODLM_EPI_STORE_F32) {
+    const int64_t c = splitk_count(M, N, K), b = use_big(M, N, K) ? gemm_big_splits(M, N, K) : 1;
+    const int64_t d = dl_ok ? gemm_dl_splits(M, N, K) : 1;
+    s = c > s ? c : s;
     s = b > s ? b : s;
-  }
-  if (M >= 256 && N >= 256 && K % 32 == 0) {
-    const int64_t d = gemm_dl_splits(M, N, K);
     s = d > s ? d : s;
   }
   return s > 1 ? s * M * N : 0;
@@ -440,26 +500,43 @@ extern "C" int alodlm_gemm(const void* A, int64_t lda, int a_kmajor, const void*
   ALODLM_CHECK_ARG(epilogue != ALODLM_EPI_RESIDUAL || R != nullptr, "gemm: residual needs R");
   if (M == 0 || N == 0) return ALODLM_OK;
   hipStream_t st = as_stream(stream);
-  if ((dtype == ALODLM_BF16 || dtype == ALODLM_F32) &&
+  const bool dl_ok = dtype == ALODLM_BF16 &&
+                     mfma_eligible(A, lda, a_kmajor, B, ldb, b_kmajor, M, N, K) &&
+                     gemm_dl_eligible(lda, a_kmajor, ldb, b_kmajor, M, N, K);
+  const bool mid_ok = dtype == ALODLM_BF16 &&
+                      gemm_mid_eligible(A, lda, a_kmajor, B, ldb, b_kmajor, M, N, K);
+  // few rows: up to one 16-row block stream the weight without LDS; above that
+  // the bf16 tiles of 32 or 64 rows, which share A between their waves, are as
+  // fast or faster (27 rows, 4096 x 12288: 27 us against 38; 4096 x 4096: 12.2
+  // against 13.5; 16 rows, 4096 x 2048: 9.6 against 6.3)
+  if ((dtype == ALODLM_F32 || (dtype == ALODLM_BF16 && (M <= 16 || !mid_ok))) &&
       gemm_skinny_eligible(A, lda, a_kmajor, B, ldb, b_kmajor, M, N, K, epilogue, dtype)) {
     gemm_skinny_launch(A, lda, B, ldb, C, ldc, R, ldr, M, N, K, alpha, epilogue, dtype, st);
     ALODLM_CHECK_LAUNCH("gemm_skinny");
     return ALODLM_OK;
   }
-  if (dtype == ALODLM_BF16 && mfma_eligible(A, lda, a_kmajor, B, ldb, b_kmajor, M, N, K) &&
-      gemm_dl_eligible(lda, a_kmajor, ldb, b_kmajor, M, N, K)) {
-    int64_t splits = 1;
-    if (epilogue == ALODLM_EPI_ACCUM || epilogue == ALODLM_EPI_STORE_F32)
-      splits = gemm_dl_splits(M, N, K);
-    else if (epilogue == ALODLM_EPI_STORE) splits = gemm_dl_store_splits(M, N, K);
-    if (splits > 1 && workspace == nullptr) splits = 1;
+  const Bf16Plan plan = bf16_plan(M, N, K, epilogue, a_kmajor, dl_ok, mid_ok, workspace != nullptr);
+  if (mid_ok && plan.mid) {
+    const int64_t nsplit = gemm_mid_launch((const bf16_t*)A, lda, a_kmajor, (const bf16_t*)B, ldb,
+                                           b_kmajor, C, ldc, (const bf16_t*)R, ldr, M, N, K, alpha,
+                                           epilogue, plan.splits, workspace, st);
+    ALODLM_CHECK_LAUNCH("gemm_bf16_mid");
+    if (nsplit > 1) {
+      splitk_reduce(workspace, nsplit, M, N, C, ldc, R, ldr, epilogue, dtype, st);
+      ALODLM_CHECK_LAUNCH("gemm_splitk_reduce");
+    }
+    return ALODLM_OK;
+  }
+  if (dl_ok) {
+    int64_t splits = plan.splits;
     if (splits > 1) {  // the launch splits K into chunks of whole 32-deep stages
       const int64_t kps = (((K + splits - 1) / splits) + 31) / 32 * 32;
       if ((K + kps - 1) / kps < 2) splits = 1;
     }
-    // a split STORE product writes float partials (the ACCUM kernel with a
-    // partial buffer), then one reduction rounds their sum to bf16
-    const int launch_epi = (epilogue == ALODLM_EPI_STORE && splits > 1) ? ALODLM_EPI_ACCUM : epilogue;
+    // a split product with a bf16 output writes float partials (the ACCUM
+    // kernel with a partial buffer), then one reduction rounds their sum
+    const bool half_out = epilogue == ALODLM_EPI_STORE || epilogue == ALODLM_EPI_RESIDUAL;
+    const int launch_epi = half_out && splits > 1 ? ALODLM_EPI_ACCUM : epilogue;
     int64_t nsplit = 1;
     // an accumulated product's split 0 adds into C in its own epilogue, so the
     // reduction reads one partial plane fewer: C = (C + p0) + (p1 + ... )
@@ -472,7 +549,7 @@ extern "C" int alodlm_gemm(const void* A, int64_t lda, int a_kmajor, const void*
       if (first_into_c)
         splitk_reduce(workspace + M * N, nsplit - 1, M, N, C, ldc, nullptr, 0, epilogue, dtype, st);
       else
-        splitk_reduce(workspace, nsplit, M, N, C, ldc, nullptr, 0, epilogue, dtype, st);
+        splitk_reduce(workspace, nsplit, M, N, C, ldc, R, ldr, epilogue, dtype, st);
       ALODLM_CHECK_LAUNCH("gemm_splitk_reduce");
     }
     return ALODLM_OK;
