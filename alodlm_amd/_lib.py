@@ -31,6 +31,7 @@ SIGNATURES = {
     "alodlm_batch_build": [P, P, P, P, I64, I64, I64, I64, P, P, P, P, P, P, P, P, P, P, P, P, P],
     "alodlm_embed_gather": [P, P, P, I64, I64, I64, I32, P],
     "alodlm_embed_plan": [P, I64, I64, P, P],
+    "alodlm_embed_scatter": [P, P, P, I64, P, P, I64, I64, I64, I32, P],
     "alodlm_embed_scatter_add": [P, P, P, I64, P, P, I64, I64, I64, I32, P],
     "alodlm_rmsnorm_fwd": [P, P, P, P, I64, I64, F32, I32, P],
     "alodlm_rmsnorm_bwd_workspace": [I64, I64],

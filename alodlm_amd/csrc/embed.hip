@@ -208,11 +208,13 @@ embed_plan_kernel(const int64_t* __restrict__ ids, int64_t n, int64_t vocab, int
 
 // One workgroup per chunk (grid.x: an upper bound, extra groups exit), W
 // columns per thread (8 with 16-byte loads when hidden % 8 == 0).
-template <typename T, int W>
+// TD: the table's type (float, or the storage type for a table that starts as
+// zeros: each row is added once, so its sum is rounded once).
+template <typename T, int W, typename TD>
 __global__ void __launch_bounds__(256)
 embed_chunk_kernel(const T* __restrict__ dout, const int32_t* __restrict__ plan, int64_t n,
                    const int32_t* __restrict__ row_exits, int64_t max_exit,
-                   float* __restrict__ dtable, float* __restrict__ partial, int64_t H,
+                   TD* __restrict__ dtable, float* __restrict__ partial, int64_t H,
                    int64_t vocab, int64_t max_slots) {
   Plan P = plan_view(const_cast<int32_t*>(plan), n);
   const int64_t c = blockIdx.x;
@@ -247,21 +249,22 @@ embed_chunk_kernel(const T* __restrict__ dout, const int32_t* __restrict__ plan,
     if constexpr (W == 8) Vec8<float>::store(dst, acc);
     else dst[0] = acc[0];
   } else if (any) {  // the run's only chunk: the only writer of this table row
-    float* dst = dtable + (int64_t)key * H + col;
+    TD* dst = dtable + (int64_t)key * H + col;
     if constexpr (W == 8) {
       float cur[8];
-      Vec8<float>::load(dst, cur);
+      Vec8<TD>::load(dst, cur);
 #pragma unroll
       for (int i = 0; i < 8; ++i) cur[i] += acc[i];
-      Vec8<float>::store(dst, cur);
+      Vec8<TD>::store(dst, cur);
     } else {
-      dst[0] += acc[0];
+      Elem<TD>::store(dst, 0, Elem<TD>::load(dst, 0) + acc[0]);
     }
   }
 }
 
+template <typename TD>
 __global__ void __launch_bounds__(256)
-embed_run_kernel(const int32_t* __restrict__ plan, int64_t n, float* __restrict__ dtable,
+embed_run_kernel(const int32_t* __restrict__ plan, int64_t n, TD* __restrict__ dtable,
                  const float* __restrict__ partial, int64_t H, int64_t vocab, int64_t max_slots) {
   Plan P = plan_view(const_cast<int32_t*>(plan), n);
   const int64_t m = blockIdx.x;
@@ -273,7 +276,8 @@ embed_run_kernel(const int32_t* __restrict__ plan, int64_t n, float* __restrict_
   if (key < 0 || key >= vocab || s0 < 0 || s1 > max_slots) return;
   float acc = 0.f;
   for (int32_t s = s0; s < s1; ++s) acc += partial[(int64_t)s * H + col];
-  dtable[(int64_t)key * H + col] += acc;
+  TD* dst = dtable + (int64_t)key * H + col;
+  Elem<TD>::store(dst, 0, Elem<TD>::load(dst, 0) + acc);
 }
 
 }  // namespace
@@ -298,30 +302,50 @@ extern "C" int64_t alodlm_embed_scatter_workspace(int64_t rows, int64_t hidden) 
   return (2 * rows / EP_CHUNK + 1) * hidden;
 }
 
+template <typename T, typename TD>
+static int scatter_launch(const T* dout, const int32_t* plan, const int32_t* row_exits,
+                          int64_t max_exit, TD* dtable, float* workspace, int64_t rows,
+                          int64_t hidden, int64_t vocab, int dtype, hipStream_t st) {
+  const int64_t max_slots = alodlm_embed_scatter_workspace(rows, hidden) / hidden;
+  const bool v8 = hidden % 8 == 0 && aligned8(dout, dtype) &&
+                  reinterpret_cast<uintptr_t>(dtable) % (8 * sizeof(TD)) == 0 &&
+                  reinterpret_cast<uintptr_t>(workspace) % 32 == 0;
+  if (v8)
+    embed_chunk_kernel<T, 8, TD><<<dim3((unsigned)rows, ceil_div_u(hidden, 256 * 8)), 256, 0, st>>>(
+        dout, plan, rows, row_exits, max_exit, dtable, workspace, hidden, vocab, max_slots);
+  else
+    embed_chunk_kernel<T, 1, TD><<<dim3((unsigned)rows, ceil_div_u(hidden, 256)), 256, 0, st>>>(
+        dout, plan, rows, row_exits, max_exit, dtable, workspace, hidden, vocab, max_slots);
+  ALODLM_CHECK_LAUNCH("embed_scatter_chunks");
+  embed_run_kernel<TD><<<dim3((unsigned)(rows / (EP_CHUNK + 1) + 1), ceil_div_u(hidden, 256)), 256,
+                         0, st>>>(plan, rows, dtable, workspace, hidden, vocab, max_slots);
+  ALODLM_CHECK_LAUNCH("embed_scatter_runs");
+  return ALODLM_OK;
+}
+
 int embed_scatter_launch(const void* dout, const int32_t* plan, const int32_t* row_exits,
                          int64_t max_exit, float* dtable, float* workspace, int64_t rows,
                          int64_t hidden, int64_t vocab, int dtype, hipStream_t st) {
   ALODLM_CHECK_ARG(rows >= 0 && rows < EP_MAX_ROWS && hidden > 0,
                    "embed_scatter_add: bad shape");
   if (rows == 0) return ALODLM_OK;
-  const int64_t max_slots = alodlm_embed_scatter_workspace(rows, hidden) / hidden;
-  const bool v8 = hidden % 8 == 0 && aligned8(dout, dtype) &&
-                  reinterpret_cast<uintptr_t>(dtable) % 32 == 0 &&
-                  reinterpret_cast<uintptr_t>(workspace) % 32 == 0;
   ALODLM_DISPATCH(dtype, T, {
-    if (v8)
-      embed_chunk_kernel<T, 8><<<dim3((unsigned)rows, ceil_div_u(hidden, 256 * 8)), 256, 0, st>>>(
-          (const T*)dout, plan, rows, row_exits, max_exit, dtable, workspace, hidden, vocab,
-          max_slots);
-    else
-      embed_chunk_kernel<T, 1><<<dim3((unsigned)rows, ceil_div_u(hidden, 256)), 256, 0, st>>>(
-          (const T*)dout, plan, rows, row_exits, max_exit, dtable, workspace, hidden, vocab,
-          max_slots);
+    return scatter_launch((const T*)dout, plan, row_exits, max_exit, dtable, workspace, rows,
+                          hidden, vocab, dtype, st);
   });
-  ALODLM_CHECK_LAUNCH("embed_scatter_chunks");
-  embed_run_kernel<<<dim3((unsigned)(rows / (EP_CHUNK + 1) + 1), ceil_div_u(hidden, 256)), 256, 0,
-                     st>>>(plan, rows, dtable, workspace, hidden, vocab, max_slots);
-  ALODLM_CHECK_LAUNCH("embed_scatter_runs");
+  return ALODLM_OK;
+}
+
+extern "C" int alodlm_embed_scatter(const void* dout, const int32_t* plan,
+                                    const int32_t* row_exits, int64_t max_exit, void* dtable,
+                                    float* workspace, int64_t rows, int64_t hidden, int64_t vocab,
+                                    int dtype, void* stream) {
+  ALODLM_CHECK_ARG(rows >= 0 && rows < EP_MAX_ROWS && hidden > 0, "embed_scatter: bad shape");
+  if (rows == 0) return ALODLM_OK;
+  ALODLM_DISPATCH(dtype, T, {
+    return scatter_launch((const T*)dout, plan, row_exits, max_exit, (T*)dtable, workspace, rows,
+                          hidden, vocab, dtype, as_stream(stream));
+  });
   return ALODLM_OK;
 }
 

@@ -568,10 +568,13 @@ extern "C" int alodlm_carry_select_bwd(const void* dy, const void* x, const floa
                                        void* stream) {
   const hipStream_t st = as_stream(stream);
   // re-embedded rows (exits <= depth) send their gradient to the embedding table
-  int rc = embed_scatter_launch(dy, plan, exits, depth, dtable,
-                                workspace + carry_norm_workspace(rows, hidden), rows, hidden,
-                                vocab, dtype, st);
-  if (rc) return rc;
+  // (unless the caller scatters them itself: no table)
+  if (dtable != nullptr) {
+    const int rc = embed_scatter_launch(dy, plan, exits, depth, dtable,
+                                        workspace + carry_norm_workspace(rows, hidden), rows,
+                                        hidden, vocab, dtype, st);
+    if (rc) return rc;
+  }
   // carried rows go back through the carry norm into the previous depth's core output
   return rmsnorm_bwd_launch(dy, x, rstd, wf, dres, dx, dwf_accum, workspace, rows, hidden, dtype,
                             exits, depth, st);

@@ -274,9 +274,12 @@ def _stack_rows(*ts):
 
 
 class LayerGrads:
-    """float32 gradient views of one layer (same layout as LayerWeights)."""
+    """Gradient views of one layer (same layout as LayerWeights), float32; with
+    ``stored`` the four projection matrices' are in the storage dtype and
+    written once (one product, rounded once) instead of accumulated."""
 
-    def __init__(self, wqkv, wo, wgu, wd, ln1, ln2, qn, kn):
+    def __init__(self, wqkv, wo, wgu, wd, ln1, ln2, qn, kn, stored=False):
+        self.stored = stored
         self.wqkv, self.wo, self.wgu, self.wd = wqkv, wo, wgu, wd
         self.ln1, self.ln2, self.qn, self.kn = ln1, ln2, qn, kn
 
@@ -445,7 +448,7 @@ class Kernels:
         and the tensors stay alive through the list."""
         _, x, rstd1, qkv, o, lse, x1, rstd2, gu, q, k, h1, h2 = saved
         d, N, st, c = self.dims, x.shape[0], self._stream(), self.code
-        wepi = EPI_STORE_F32 if first else EPI_ACCUM
+        wepi = EPI_STORE if gw.stored else EPI_STORE_F32 if first else EPI_ACCUM
 
         def dw(A, lda, B, ldb, C, ldc, M, Nc):  # C (+)= A^T B over the N rows
             if defer is None:
@@ -618,20 +621,19 @@ class _LayerFunction(torch.autograd.Function):
     def backward(ctx, dy, _dk, _dv):
         kernels, w, d = ctx.kernels, ctx.w, ctx.kernels.dims
         H, W, I, QD = d.hidden, d.qkv_width, d.intermediate, d.heads * d.head_dim
-        sizes = [W * H, H * QD, 2 * I * H, H * I, H, H, d.head_dim, d.head_dim]
-        flat = torch.zeros(sum(sizes), dtype=torch.float32, device=kernels.device)
-        views, off = [], 0
-        for n in sizes:
-            views.append(flat[off:off + n])
-            off += n
-        gw = LayerGrads(views[0].view(W, H), views[1].view(H, QD), views[2].view(2 * I, H),
-                        views[3].view(H, I), *views[4:])
+        # the matrices' gradients in the parameter dtype, written by their
+        # products; the norm weights' sums in float32
+        mats = kernels._empty(W * H + H * QD + 3 * I * H).split([W * H, H * QD, 2 * I * H, H * I])
+        norms = torch.zeros(2 * H + 2 * d.head_dim, dtype=torch.float32, device=kernels.device)
+        gw = LayerGrads(mats[0].view(W, H), mats[1].view(H, QD), mats[2].view(2 * I, H),
+                        mats[3].view(H, I), *norms.split([H, H, d.head_dim, d.head_dim]),
+                        stored=True)
         dx = kernels.layer_bwd(dy.contiguous(), ctx.saved, w, gw, ctx.mask, ctx.rope)
         ctx.saved = None
         qd, kd = QD, d.kv_heads * d.head_dim
         parts = [gw.wqkv[:qd], gw.wqkv[qd:qd + kd], gw.wqkv[qd + kd:], gw.wo, gw.wgu[:I],
                  gw.wgu[I:], gw.wd, gw.ln1, gw.ln2, gw.qn, gw.kn]
-        grads = [g.reshape(shape).to(dtype) for g, (shape, dtype) in zip(parts, ctx.shapes)]
+        grads = [g.view(shape).to(dtype) for g, (shape, dtype) in zip(parts, ctx.shapes)]
         return (None, None, None, dx, *grads)
 
 

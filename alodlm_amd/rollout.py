@@ -17,12 +17,24 @@ the loss-bearing rows' logits.
 import torch
 
 from . import _lib
-from ._lib import EPI_ACCUM, call, ptr, query
+from ._lib import call, ptr, query
 from .layers import DualStreamMask, LayerWeights, Rope, _LayerFunction
 
 
 def _f32_zeros(*shape, device):
     return torch.zeros(*shape, dtype=torch.float32, device=device)
+
+
+def _table_grad(k, dout, ids, vocab, row_exits=None, max_exit=0):
+    """The gradient [vocab, hidden] of an embedding gather in the parameter
+    dtype (each row's sum in float32, rounded once), over all rows or those
+    with row_exits[r] <= max_exit."""
+    N, H = dout.shape
+    table = torch.zeros(vocab, H, dtype=k.dtype, device=k.device)
+    ws = k._workspace(query("alodlm_embed_scatter_workspace", N, H))
+    call("alodlm_embed_scatter", ptr(dout), ptr(k.embed_plan(ids)), ptr(row_exits), max_exit,
+         ptr(table), ptr(ws), N, H, vocab, k.code, k._stream())
+    return table
 
 
 class _Embedding(torch.autograd.Function):
@@ -38,9 +50,7 @@ class _Embedding(torch.autograd.Function):
     @staticmethod
     def backward(ctx, dout):
         k, (V, H) = ctx.kernels, ctx.shape
-        dtable = _f32_zeros(V, H, device=k.device)
-        k.embed_scatter(dout.contiguous(), k.embed_plan(ctx.ids), dtable)
-        return None, None, dtable.to(k.dtype)
+        return None, None, _table_grad(k, dout.contiguous(), ctx.ids, V)
 
 
 class _CarrySelect(torch.autograd.Function):
@@ -69,12 +79,13 @@ class _CarrySelect(torch.autograd.Function):
         V = ctx.vocab
         dx = k._empty(N, H)
         dwf = _f32_zeros(H, device=k.device)
-        dtable = _f32_zeros(V, H, device=k.device)
+        dy = dy.contiguous()
+        dtable = _table_grad(k, dy, ctx.original, V, ctx.exits, ctx.depth)
         ws = k._workspace(query("alodlm_carry_select_bwd_workspace", N, H))
-        call("alodlm_carry_select_bwd", ptr(dy.contiguous()), ptr(core_out), ptr(rstd), ptr(wf),
-             ptr(ctx.exits), ctx.depth, ptr(k.embed_plan(ctx.original)), None, ptr(dx), ptr(dwf),
-             ptr(dtable), ptr(ws), N, H, V, k.code, k._stream())
-        return None, None, None, None, dx, dwf.to(k.dtype), dtable.to(k.dtype)
+        call("alodlm_carry_select_bwd", ptr(dy), ptr(core_out), ptr(rstd), ptr(wf),
+             ptr(ctx.exits), ctx.depth, None, None, ptr(dx), ptr(dwf), None, ptr(ws), N, H, V,
+             k.code, k._stream())
+        return None, None, None, None, dx, dwf.to(k.dtype), dtable
 
 
 class _FinalNormGate(torch.autograd.Function):
@@ -143,9 +154,9 @@ class _LMHead(torch.autograd.Function):
         dy = dy.contiguous()
         dx = k._empty(N, H)
         k._gemm(dy, V, 1, w, H, 0, dx, H, N, H, V)
-        dw = _f32_zeros(V, H, device=k.device)
-        k._gemm(dy, V, 0, x, H, 0, dw, H, V, H, N, epi=EPI_ACCUM)
-        return None, dx, dw.to(k.dtype)
+        dw = k._empty(V, H)
+        k._gemm(dy, V, 0, x, H, 0, dw, H, V, H, N)
+        return None, dx, dw
 
 
 def _mask_of(batch, device):

@@ -106,6 +106,12 @@ int64_t alodlm_embed_scatter_workspace(int64_t rows, int64_t hidden);
 int alodlm_embed_scatter_add(const void* dout, const int32_t* plan, const int32_t* row_exits,
                              int64_t max_exit, float* dtable, float* workspace, int64_t rows,
                              int64_t hidden, int64_t vocab, int dtype, void* stream);
+/* The same into a table [vocab, hidden] of the storage type, which must hold
+ * zeros: every row's sum is taken in float32 and rounded once. */
+int alodlm_embed_scatter(const void* dout, const int32_t* plan, const int32_t* row_exits,
+                         int64_t max_exit, void* dtable, float* workspace, int64_t rows,
+                         int64_t hidden, int64_t vocab, int dtype, void* stream);
+
 
 /* ---------------------------------------------------------------------------
  * RMSNorm ([tf] modeling_qwen3.py:59-64): y = w * cast(x * rsqrt(mean(x^2) + eps)).
