@@ -222,21 +222,28 @@ __device__ __forceinline__ float sum8(float v) {
   return v;
 }
 
+template <bool TAB>
 __global__ void __launch_bounds__(64 * ROPE_WAVES)
 qknorm_rope128_fwd_kernel(const bf16_t* __restrict__ qkv, const bf16_t* __restrict__ wq,
                           const bf16_t* __restrict__ wk, const int64_t* __restrict__ positions,
-                          const float* __restrict__ inv_freq, bf16_t* __restrict__ q_out,
+                          const float* __restrict__ inv_freq, const bf16_t* __restrict__ cos_tab,
+                          const bf16_t* __restrict__ sin_tab, bf16_t* __restrict__ q_out,
                           bf16_t* __restrict__ k_out, int64_t rows, int nq, int nkv, float eps) {
   const int lane = threadIdx.x & 63, slot = lane >> 3, j = lane & 7;
   const int64_t row = (int64_t)blockIdx.x * ROPE_WAVES + (threadIdx.x >> 6);
   if (row >= rows) return;
   const int i0 = 8 * j;
-  const float pos = (float)positions[row];
-  // lane l computes the rotation of frequency l; lane j of a head takes
-  // frequencies 8j..8j+7 from lanes 8j..8j+7
-  float cs[8], sn[8], wqa[8], wqb[8], wka[8], wkb[8];
-  {
-    const float ang = pos * inv_freq[lane];
+  // from positions, both halves of a pair share one angle: lane l computes the
+  // rotation of frequency l and lane j of a head takes frequencies 8j..8j+7
+  // from lanes 8j..8j+7; from tables each half has its own entries
+  float cs[8], sn[8], cb_[TAB ? 8 : 1], sb_[TAB ? 8 : 1], wqa[8], wqb[8], wka[8], wkb[8];
+  if constexpr (TAB) {
+    Vec8<bf16_t>::load(cos_tab + row * 128 + i0, cs);
+    Vec8<bf16_t>::load(sin_tab + row * 128 + i0, sn);
+    Vec8<bf16_t>::load(cos_tab + row * 128 + i0 + 64, cb_);
+    Vec8<bf16_t>::load(sin_tab + row * 128 + i0 + 64, sb_);
+  } else {
+    const float ang = (float)positions[row] * inv_freq[lane];
     const float c1 = round_bf16(cosf(ang)), s1 = round_bf16(sinf(ang));
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
@@ -244,11 +251,13 @@ qknorm_rope128_fwd_kernel(const bf16_t* __restrict__ qkv, const bf16_t* __restri
       sn[e] = __shfl(s1, i0 + e, 64);
     }
   }
+  const float* cb = TAB ? cb_ : cs;
+  const float* sb = TAB ? sb_ : sn;
   Vec8<bf16_t>::load(wq + i0, wqa); Vec8<bf16_t>::load(wq + i0 + 64, wqb);
   Vec8<bf16_t>::load(wk + i0, wka); Vec8<bf16_t>::load(wk + i0 + 64, wkb);
   const int heads = nq + nkv;
   const bf16_t* src = qkv + row * (int64_t)(nq + 2 * nkv) * 128;
-  for (int h0 = 0; h0 < heads; h0 += 8) {
+  for (int h0 = 8 * blockIdx.y; h0 < heads; h0 += 8 * gridDim.y) {
     const int head = h0 + slot;
     const bool live = head < heads;
     const bool is_q = head < nq;
@@ -267,7 +276,7 @@ qknorm_rope128_fwd_kernel(const bf16_t* __restrict__ qkv, const bf16_t* __restri
       const float a = round_bf16((is_q ? wqa[e] : wka[e]) * round_bf16(xa[e] * r));
       const float b = round_bf16((is_q ? wqb[e] : wkb[e]) * round_bf16(xb[e] * r));
       oa[e] = round_bf16(a * cs[e]) + round_bf16(-b * sn[e]);
-      ob[e] = round_bf16(b * cs[e]) + round_bf16(a * sn[e]);
+      ob[e] = round_bf16(b * cb[e]) + round_bf16(a * sb[e]);
     }
     if (live) {
       bf16_t* dst = is_q ? q_out + (row * nq + head) * 128 : k_out + (row * nkv + head - nq) * 128;
@@ -277,18 +286,20 @@ qknorm_rope128_fwd_kernel(const bf16_t* __restrict__ qkv, const bf16_t* __restri
   }
 }
 
+template <bool TAB>
 __global__ void __launch_bounds__(64 * ROPE_WAVES)
 qknorm_rope128_bwd_kernel(const bf16_t* __restrict__ dq, const bf16_t* __restrict__ dk,
                           const bf16_t* __restrict__ qkv, const bf16_t* __restrict__ wq,
                           const bf16_t* __restrict__ wk, const int64_t* __restrict__ positions,
-                          const float* __restrict__ inv_freq, bf16_t* __restrict__ dqkv,
+                          const float* __restrict__ inv_freq, const bf16_t* __restrict__ cos_tab,
+                          const bf16_t* __restrict__ sin_tab, bf16_t* __restrict__ dqkv,
                           float* __restrict__ partial, int64_t rows, int nq, int nkv, float eps,
                           int64_t rows_per_block) {
   __shared__ float lds[ROPE_WAVES * 4][2 * 128];  // [wave*4 + slot][dwq | dwk]
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, slot = lane >> 4, j = lane & 15;
   const int i0 = 4 * j;
   const int64_t width = (int64_t)(nq + 2 * nkv) * 128;
-  const float freq = inv_freq[lane];
+  const float freq = TAB ? 0.f : inv_freq[lane];
   const int64_t r0 = (int64_t)blockIdx.x * rows_per_block;
   float* L = lds[wave * 4 + slot];
   // the q heads of the block's rows, then the k heads: one weight-gradient
@@ -300,10 +311,13 @@ qknorm_rope128_bwd_kernel(const bf16_t* __restrict__ dq, const bf16_t* __restric
     float wa[4], wb[4], ga[4] = {0.f, 0.f, 0.f, 0.f}, gb[4] = {0.f, 0.f, 0.f, 0.f};
     load4(w + i0, wa); load4(w + i0 + 64, wb);
     for (int64_t row = r0 + wave; row < r0 + rows_per_block && row < rows; row += ROPE_WAVES) {
-      // lane l computes the rotation of frequency l; lane j of a head takes
-      // frequencies 4j..4j+3 from lanes 4j..4j+3
-      float cs[4], sn[4];
-      {
+      // (positions) lane l computes the rotation of frequency l; lane j of a
+      // head takes frequencies 4j..4j+3 from lanes 4j..4j+3
+      float cs[4], sn[4], cb_[TAB ? 4 : 1], sb_[TAB ? 4 : 1];
+      if constexpr (TAB) {
+        load4(cos_tab + row * 128 + i0, cs); load4(cos_tab + row * 128 + i0 + 64, cb_);
+        load4(sin_tab + row * 128 + i0, sn); load4(sin_tab + row * 128 + i0 + 64, sb_);
+      } else {
         const float ang = (float)positions[row] * freq;
         const float c1 = round_bf16(cosf(ang)), s1 = round_bf16(sinf(ang));
 #pragma unroll
@@ -312,6 +326,8 @@ qknorm_rope128_bwd_kernel(const bf16_t* __restrict__ dq, const bf16_t* __restric
           sn[e] = __shfl(s1, i0 + e, 64);
         }
       }
+      const float* cb = TAB ? cb_ : cs;
+      const float* sb = TAB ? sb_ : sn;
       for (int h0 = h_beg; h0 < h_end; h0 += 4) {
         const int head = h0 + slot;
         const bool live = head < h_end;
@@ -326,8 +342,8 @@ qknorm_rope128_bwd_kernel(const bf16_t* __restrict__ dq, const bf16_t* __restric
         float ta[4], tb[4], ss = 0.f, s = 0.f;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          ta[e] = go[e] * cs[e] + gh[e] * sn[e];   // d/d t[i]
-          tb[e] = gh[e] * cs[e] - go[e] * sn[e];   // d/d t[i + half]
+          ta[e] = go[e] * cs[e] + gh[e] * sb[e];   // d/d t[i]
+          tb[e] = gh[e] * cb[e] - go[e] * sn[e];   // d/d t[i + half]
           ss += xa[e] * xa[e] + xb[e] * xb[e];
           s += ta[e] * wa[e] * xa[e] + tb[e] * wb[e] * xb[e];
         }
@@ -377,6 +393,15 @@ static bool rope128_aligned16(const void* a, const void* b, const void* c) {
            reinterpret_cast<uintptr_t>(c)) & 15) == 0;
 }
 
+// Head groups of 8 per row in the head_dim-128 forward: one wavefront walks a
+// row's groups where the rows alone fill the chip (four wavefronts per SIMD),
+// else each group gets its own (a decoder window's 16 rows of 24 heads: three
+// short walks side by side instead of one of three).
+static dim3 rope128_grid(int64_t rows, int64_t nq, int64_t nkv) {
+  const unsigned groups = rows < 4096 ? ceil_div_u(nq + nkv, 8) : 1;
+  return dim3(ceil_div_u(rows, ROPE_WAVES), groups < 65535 ? groups : 65535);
+}
+
 static int check_rope(int64_t rows, int64_t nq, int64_t nkv, int64_t dh) {
   ALODLM_CHECK_ARG(rows >= 0 && nq > 0 && nkv > 0, "qknorm_rope: bad head counts");
   ALODLM_CHECK_ARG(dh > 0 && dh % 2 == 0 && dh <= 128 * ROPE_MAX_T,
@@ -394,10 +419,10 @@ extern "C" int alodlm_qknorm_rope_fwd(const void* qkv, const void* wq, const voi
   ALODLM_DISPATCH(dtype, T, {
     if (std::is_same<T, bf16_t>::value && dh == 128 && rope128_aligned16(qkv, q_out, k_out) &&
         rope128_aligned16(wq, wk, wk)) {
-      qknorm_rope128_fwd_kernel<<<ceil_div_u(rows, ROPE_WAVES), 64 * ROPE_WAVES, 0,
-                                  as_stream(stream)>>>(
-          (const bf16_t*)qkv, (const bf16_t*)wq, (const bf16_t*)wk, positions, inv_freq,
-          (bf16_t*)q_out, (bf16_t*)k_out, rows, (int)nq, (int)nkv, eps);
+      qknorm_rope128_fwd_kernel<false><<<rope128_grid(rows, nq, nkv), 64 * ROPE_WAVES, 0,
+                                         as_stream(stream)>>>(
+          (const bf16_t*)qkv, (const bf16_t*)wq, (const bf16_t*)wk, positions, inv_freq, nullptr,
+          nullptr, (bf16_t*)q_out, (bf16_t*)k_out, rows, (int)nq, (int)nkv, eps);
       break;
     }
     qknorm_rope_fwd_kernel<T, false><<<ceil_div_u(rows, ROPE_WAVES), 64 * ROPE_WAVES, 0,
@@ -409,12 +434,24 @@ extern "C" int alodlm_qknorm_rope_fwd(const void* qkv, const void* wq, const voi
   return ALODLM_OK;
 }
 
+// The blocks' partial rows [dwq | dwk] into the two gradients: one launch where
+// they are adjacent (as the step's arena and the layer function lay them out).
+static int reduce_norm_grads(float* workspace, int64_t nparts, int64_t dh, float* dwq_accum,
+                             float* dwk_accum, hipStream_t st) {
+  float* tmp = workspace + nparts * 2 * dh;
+  if (dwk_accum == dwq_accum + dh)
+    return column_reduce(workspace, nparts, 2 * dh, 0, 2 * dh, dwq_accum, tmp, st);
+  const int rc = column_reduce(workspace, nparts, 2 * dh, 0, dh, dwq_accum, tmp, st);
+  if (rc) return rc;
+  return column_reduce(workspace, nparts, 2 * dh, dh, dh, dwk_accum, tmp, st);
+}
+
 extern "C" int64_t alodlm_qknorm_rope_bwd_workspace(int64_t rows, int64_t nq, int64_t nkv,
                                                     int64_t dh) {
   (void)nq; (void)nkv;
   // per-block partial rows [dwq | dwk], then the column reduction's group sums
   const int64_t rpb = bwd_rows_per_block(rows);
-  return ((rows + rpb - 1) / rpb) * 2 * dh + COLUMN_REDUCE_MAX_GROUPS * dh;
+  return ((rows + rpb - 1) / rpb) * 2 * dh + COLUMN_REDUCE_MAX_GROUPS * 2 * dh;
 }
 
 extern "C" int alodlm_qknorm_rope_bwd(const void* dq, const void* dk, const void* qkv,
@@ -431,9 +468,9 @@ extern "C" int alodlm_qknorm_rope_bwd(const void* dq, const void* dk, const void
   ALODLM_DISPATCH(dtype, T, {
     if (std::is_same<T, bf16_t>::value && dh == 128 && rope128_aligned(dq, dk, qkv) &&
         rope128_aligned(dqkv, wq, wk)) {
-      qknorm_rope128_bwd_kernel<<<(unsigned)nparts, 64 * ROPE_WAVES, 0, st>>>(
+      qknorm_rope128_bwd_kernel<false><<<(unsigned)nparts, 64 * ROPE_WAVES, 0, st>>>(
           (const bf16_t*)dq, (const bf16_t*)dk, (const bf16_t*)qkv, (const bf16_t*)wq,
-          (const bf16_t*)wk, positions, inv_freq, (bf16_t*)dqkv, workspace, rows, (int)nq,
+          (const bf16_t*)wk, positions, inv_freq, nullptr, nullptr, (bf16_t*)dqkv, workspace, rows, (int)nq,
           (int)nkv, eps, rpb);
       break;
     }
@@ -444,10 +481,7 @@ extern "C" int alodlm_qknorm_rope_bwd(const void* dq, const void* dk, const void
         rpb);
   });
   ALODLM_CHECK_LAUNCH("qknorm_rope_bwd");
-  float* tmp = workspace + nparts * 2 * dh;
-  rc = column_reduce(workspace, nparts, 2 * dh, 0, dh, dwq_accum, tmp, st);
-  if (rc) return rc;
-  return column_reduce(workspace, nparts, 2 * dh, dh, dh, dwk_accum, tmp, st);
+  return reduce_norm_grads(workspace, nparts, dh, dwq_accum, dwk_accum, st);
 }
 
 // ---------------------------------------------------------------------------
@@ -462,6 +496,15 @@ extern "C" int alodlm_qknorm_rotary_fwd(const void* qkv, const void* wq, const v
   if (rc) return rc;
   if (rows == 0) return ALODLM_OK;
   ALODLM_DISPATCH(dtype, T, {
+    if (std::is_same<T, bf16_t>::value && dh == 128 && rope128_aligned16(qkv, q_out, k_out) &&
+        rope128_aligned16(wq, wk, wk) && rope128_aligned16(cos_tab, sin_tab, sin_tab)) {
+      qknorm_rope128_fwd_kernel<true><<<rope128_grid(rows, nq, nkv), 64 * ROPE_WAVES, 0,
+                                        as_stream(stream)>>>(
+          (const bf16_t*)qkv, (const bf16_t*)wq, (const bf16_t*)wk, nullptr, nullptr,
+          (const bf16_t*)cos_tab, (const bf16_t*)sin_tab, (bf16_t*)q_out, (bf16_t*)k_out, rows,
+          (int)nq, (int)nkv, eps);
+      break;
+    }
     qknorm_rope_fwd_kernel<T, true><<<ceil_div_u(rows, ROPE_WAVES), 64 * ROPE_WAVES, 0,
                                       as_stream(stream)>>>(
         (const T*)qkv, (const T*)wq, (const T*)wk, nullptr, nullptr, (const T*)cos_tab,
@@ -484,6 +527,14 @@ extern "C" int alodlm_qknorm_rotary_bwd(const void* dq, const void* dk, const vo
   const int64_t nparts = (rows + rpb - 1) / rpb;
   hipStream_t st = as_stream(stream);
   ALODLM_DISPATCH(dtype, T, {
+    if (std::is_same<T, bf16_t>::value && dh == 128 && rope128_aligned(dq, dk, qkv) &&
+        rope128_aligned(dqkv, wq, wk) && rope128_aligned(cos_tab, sin_tab, sin_tab)) {
+      qknorm_rope128_bwd_kernel<true><<<(unsigned)nparts, 64 * ROPE_WAVES, 0, st>>>(
+          (const bf16_t*)dq, (const bf16_t*)dk, (const bf16_t*)qkv, (const bf16_t*)wq,
+          (const bf16_t*)wk, nullptr, nullptr, (const bf16_t*)cos_tab, (const bf16_t*)sin_tab,
+          (bf16_t*)dqkv, workspace, rows, (int)nq, (int)nkv, eps, rpb);
+      break;
+    }
     qknorm_rope_bwd_kernel<T, true><<<(unsigned)nparts, 64 * ROPE_WAVES,
                                       ROPE_WAVES * 2 * dh * sizeof(float), st>>>(
         (const T*)dq, (const T*)dk, (const T*)qkv, (const T*)wq, (const T*)wk, nullptr, nullptr,
@@ -491,10 +542,7 @@ extern "C" int alodlm_qknorm_rotary_bwd(const void* dq, const void* dk, const vo
         (int)dh, eps, rpb);
   });
   ALODLM_CHECK_LAUNCH("qknorm_rotary_bwd");
-  float* tmp = workspace + nparts * 2 * dh;
-  rc = column_reduce(workspace, nparts, 2 * dh, 0, dh, dwq_accum, tmp, st);
-  if (rc) return rc;
-  return column_reduce(workspace, nparts, 2 * dh, dh, dh, dwk_accum, tmp, st);
+  return reduce_norm_grads(workspace, nparts, dh, dwq_accum, dwk_accum, st);
 }
 
 // out = x * cos + rotate_half(x) * sin for every head of a row, with the
