@@ -67,6 +67,8 @@ SIGNATURES = {
     "alodlm_gather_rows": [P, P, I64, P, I64, I32, P],
     "alodlm_scatter_rows": [P, P, I64, P, I64, I64, I32, P],
     "alodlm_cross_entropy": [P, P, P, P, I64, I64, P, P, I32, P],
+    "alodlm_cross_entropy_rows": [P, P, P, P, P, P, I64, I64, P, P, I32, P],
+    "alodlm_spread_rows": [P, P, I64, P, P, I64, I64, I32, P],
     "alodlm_scatter_ce": [P, P, P, I64, P, I64, P],
     "alodlm_decode_readout": [P, I64, I64, P, P, I32, P],
     "alodlm_decode_plan": [P, P],
@@ -78,6 +80,7 @@ SIGNATURES = {
     "alodlm_masked_sequence_ids": [P, P, I64, I64, P, P, P],
     "alodlm_sequence_score": [P, P, P, I64, I64, P, P, P, P],
     "alodlm_ar_targets": [P, P, I64, I64, P, P],
+    "alodlm_ar_rows": [P, P, I64, I64, P, P, P, P],
     "alodlm_gate_bwd_workspace": [I64, I64],
     "alodlm_gate_bwd": [P, P, F32, P, P, P, I64, I64, I64, P, I32, P],
     "alodlm_grad_norm": [P, P, P, P, I64, I64, I32, P, P, P],

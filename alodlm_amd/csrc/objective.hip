@@ -335,25 +335,56 @@ extern "C" int alodlm_sequence_score(const float* credit, const float* logq, con
 // for the segment with dual-stream rows [start, end) and L = (end - start)/2,
 // clean row start + i (i < L - 1) predicts labels[start/2 + 1 + i]; every
 // other row, and ignored labels (-100), get -1.
-__global__ void ar_targets_kernel(const int64_t* __restrict__ labels,
-                                  const int64_t* __restrict__ bounds, int64_t S, int64_t rows,
-                                  int32_t* __restrict__ target) {
-  const int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (r >= rows) return;
+__device__ __forceinline__ int32_t ar_target_of(const int64_t* labels, const int64_t* bounds,
+                                                int64_t S, int64_t r) {
   int64_t lo = 0, hi = S;
   while (lo < hi) {
     const int64_t mid = (lo + hi) >> 1;
     if (bounds[mid + 1] <= r) lo = mid + 1; else hi = mid;
   }
-  int32_t t = -1;
-  if (lo < S) {
-    const int64_t start = bounds[lo], L = (bounds[lo + 1] - start) / 2, i = r - start;
-    if (L >= 2 && i < L - 1) {
-      const int64_t label = labels[start / 2 + 1 + i];
-      if (label != -100) t = (int32_t)label;
+  if (lo >= S) return -1;
+  const int64_t start = bounds[lo], L = (bounds[lo + 1] - start) / 2, i = r - start;
+  if (L < 2 || i >= L - 1) return -1;
+  const int64_t label = labels[start / 2 + 1 + i];
+  return label != -100 ? (int32_t)label : -1;
+}
+
+__global__ void ar_targets_kernel(const int64_t* __restrict__ labels,
+                                  const int64_t* __restrict__ bounds, int64_t S, int64_t rows,
+                                  int32_t* __restrict__ target) {
+  const int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (r < rows) target[r] = ar_target_of(labels, bounds, S, r);
+}
+
+// The rows with a target, in order, with their targets and their number: one
+// workgroup walks the rows 1024 at a time (a pack's rows are a few thousand;
+// it replaces a compare, a two-kernel nonzero, a gather and two conversions).
+__global__ void __launch_bounds__(1024)
+ar_rows_kernel(const int64_t* __restrict__ labels, const int64_t* __restrict__ bounds, int64_t S,
+               int64_t rows, int32_t* __restrict__ sel, int32_t* __restrict__ target,
+               int32_t* __restrict__ count) {
+  __shared__ int waves[16];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  int total = 0;
+  for (int64_t r0 = 0; r0 < rows; r0 += 1024) {
+    const int64_t r = r0 + threadIdx.x;
+    const int32_t t = r < rows ? ar_target_of(labels, bounds, S, r) : -1;
+    const uint64_t live = __ballot(t >= 0);
+    if (lane == 0) waves[wave] = __popcll(live);
+    __syncthreads();
+    int before = total;
+    for (int w = 0; w < 16; ++w) {
+      if (w < wave) before += waves[w];
+      total += waves[w];
     }
+    if (t >= 0) {
+      const int at = before + __popcll(live & ((1ull << lane) - 1));
+      sel[at] = (int32_t)r;
+      target[at] = t;
+    }
+    __syncthreads();
   }
-  target[r] = t;
+  if (threadIdx.x == 0) *count = total;
 }
 
 extern "C" int alodlm_ar_targets(const int64_t* labels, const int64_t* bounds, int64_t n_segments,
@@ -363,5 +394,15 @@ extern "C" int alodlm_ar_targets(const int64_t* labels, const int64_t* bounds, i
   ar_targets_kernel<<<ceil_div_u(rows, 256), 256, 0, as_stream(stream)>>>(labels, bounds,
                                                                          n_segments, rows, target);
   ALODLM_CHECK_LAUNCH("ar_targets");
+  return ALODLM_OK;
+}
+
+extern "C" int alodlm_ar_rows(const int64_t* labels, const int64_t* bounds, int64_t n_segments,
+                              int64_t rows, int32_t* sel, int32_t* target, int32_t* count,
+                              void* stream) {
+  ALODLM_CHECK_ARG(rows >= 0 && rows < (1LL << 31) && n_segments >= 1, "ar_rows: bad shape");
+  ar_rows_kernel<<<1, 1024, 0, as_stream(stream)>>>(labels, bounds, n_segments, rows, sel, target,
+                                                    count);
+  ALODLM_CHECK_LAUNCH("ar_rows");
   return ALODLM_OK;
 }

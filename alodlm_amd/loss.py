@@ -83,22 +83,17 @@ def outcome_loss(ce, gate_logits, depths, batch, config):
 
 class _AutoregressiveLoss(torch.autograd.Function):
     @staticmethod
-    def forward(ctx, logits, rows, targets):
+    def forward(ctx, logits, sel, target, n_rows, R):
         dev, (N, V) = logits.device, logits.shape
-        R = rows.numel()
-        code, st = _lib.dtype_code(logits.dtype), _lib.stream_handle(dev)
-        sel = rows.to(torch.int32).contiguous()
         buf = torch.empty(R, V, dtype=logits.dtype, device=dev)
         src = logits.detach().contiguous()
-        call("alodlm_gather_rows", ptr(src), ptr(sel), R, ptr(buf), V, code, st)
         coef = torch.full((R,), 1.0 / R, dtype=torch.float32, device=dev)
-        n_rows = torch.full((1,), R, dtype=torch.int32, device=dev)
         ce = torch.empty(R, dtype=torch.float32, device=dev)
-        tgt = targets.to(torch.int32).contiguous()
         # ce[r] = logsumexp - logit[target]; buf <- (softmax - onehot) / R
-        call("alodlm_cross_entropy", ptr(buf), ptr(tgt), ptr(coef), ptr(n_rows), R, V, ptr(ce),
-             None, code, st)
-        ctx.save_for_backward(buf, sel)
+        call("alodlm_cross_entropy_rows", ptr(src), ptr(sel), ptr(buf), ptr(target), ptr(coef),
+             ptr(n_rows), R, V, ptr(ce), None, _lib.dtype_code(logits.dtype),
+             _lib.stream_handle(dev))
+        ctx.save_for_backward(buf, sel[:R])
         ctx.shape = (N, V)
         return ce.sum() / R
 
@@ -106,11 +101,11 @@ class _AutoregressiveLoss(torch.autograd.Function):
     def backward(ctx, grad):
         buf, sel = ctx.saved_tensors
         N, V = ctx.shape
-        scaled = (buf * grad.to(buf.dtype)).contiguous()
-        out = torch.zeros(N, V, dtype=buf.dtype, device=buf.device)
-        call("alodlm_scatter_rows", ptr(scaled), ptr(sel), sel.numel(), ptr(out), N, V,
+        out = torch.empty(N, V, dtype=buf.dtype, device=buf.device)
+        scale = grad.to(torch.float32).reshape(1)
+        call("alodlm_spread_rows", ptr(buf), ptr(sel), sel.numel(), ptr(scale), ptr(out), N, V,
              _lib.dtype_code(buf.dtype), _lib.stream_handle(buf.device))
-        return out, None, None
+        return out, None, None, None, None
 
 
 def autoregressive_loss(logits, labels, packed_boundaries):
@@ -123,10 +118,11 @@ def autoregressive_loss(logits, labels, packed_boundaries):
     N = logits.shape[0]
     bounds = packed_boundaries.to(device=logits.device, dtype=torch.int64).contiguous()
     lab = labels.to(device=logits.device, dtype=torch.int64).contiguous()
-    target = torch.empty(N, dtype=torch.int32, device=logits.device)
-    call("alodlm_ar_targets", ptr(lab), ptr(bounds), bounds.numel() - 1, N, ptr(target),
-         _lib.stream_handle(logits.device))
-    rows = torch.nonzero(target >= 0).flatten()
-    if rows.numel() == 0:
+    sel = torch.empty(2 * N + 1, dtype=torch.int32, device=logits.device)
+    target, n_rows = sel[N:2 * N], sel[2 * N:]
+    call("alodlm_ar_rows", ptr(lab), ptr(bounds), bounds.numel() - 1, N, ptr(sel), ptr(target),
+         ptr(n_rows), _lib.stream_handle(logits.device))
+    R = int(n_rows.item())
+    if R == 0:
         return torch.tensor(0.0, device=logits.device, requires_grad=True)
-    return _AutoregressiveLoss.apply(logits, rows, target[rows])
+    return _AutoregressiveLoss.apply(logits, sel, target, n_rows, R)

@@ -347,6 +347,20 @@ int alodlm_scatter_rows(const void* src, const int32_t* sel_rows, int64_t n_sel,
 int alodlm_cross_entropy(void* logits, const int32_t* target, const float* coef,
                          const int32_t* n_rows, int64_t max_rows, int64_t vocab, float* ce,
                          float* entropy, int dtype, void* stream);
+/* The same for rows src_rows[j] (j < n_rows[0] <= max_rows) of another buffer
+ * src: row j of dlogits [max_rows, vocab] receives coef[j]*(softmax - onehot),
+ * src is left unchanged, ce is the float32 cross-entropy without the storage
+ * type's rounding (alodlm/loss.py:12-32 on given logits). */
+int alodlm_cross_entropy_rows(const void* src, const int32_t* src_rows, void* dlogits,
+                              const int32_t* target, const float* coef, const int32_t* n_rows,
+                              int64_t max_rows, int64_t vocab, float* ce, float* entropy,
+                              int dtype, void* stream);
+/* dst [dst_rows, vocab]: row rows[j] = scale[0] * src row j for the n ascending
+ * row indices `rows`, every other row zero (the gradient of the above in the
+ * whole logits, times the loss's upstream gradient). */
+int alodlm_spread_rows(const void* src, const int32_t* rows, int64_t n, const float* scale,
+                       void* dst, int64_t dst_rows, int64_t vocab, int dtype, void* stream);
+
 /* Decode readout (alodlm/inference.py:115-118: logits.argmax(-1) and the
  * entropy -(exp(logp) * logp).sum(-1) of log_softmax(logits.float())):
  * logits [rows, V] (dtype, unchanged) -> argmax[rows] (int64; the first index
@@ -485,6 +499,10 @@ int alodlm_sequence_score(const float* credit, const float* logq, const int64_t*
  * every other row and ignored labels (-100) get -1. */
 int alodlm_ar_targets(const int64_t* labels, const int64_t* bounds, int64_t n_segments,
                       int64_t rows, int32_t* target, void* stream);
+/* The rows with a target in order: sel, target [rows] hold count[0] entries. */
+int alodlm_ar_rows(const int64_t* labels, const int64_t* bounds, int64_t n_segments, int64_t rows,
+                   int32_t* sel, int32_t* target, int32_t* count, void* stream);
+
 
 /* Gate-head backward (GateHead.forward, model.py:37-38, differentiated):
  * gw_accum[H] += scale * sum_r dgate[r]*readout[r]; gb_accum[0] and
