@@ -6,7 +6,8 @@
 // rows of its own block.  The kernels enumerate exactly those key ranges, so
 // no masked pair and no cross-segment pair is ever visited.
 //
-// bf16 with head_dim 64 or 128 runs attention_mfma.hip / attention_fa128.hip,
+// bf16 with head_dim 64 or 128 runs attention_mfma.hip / attention_fa128.hip
+// (few queries: attention_few.hip),
 // float with head_dim 128 attention_f32.hip.
 // Reference kernels (any dtype, any head_dim): one wavefront per (query row,
 // head) in the forward and dQ passes and one per (key row, kv head) in the
@@ -215,6 +216,9 @@ int fa128_bwd_launch(const bf16_t* q, const bf16_t* k, const bf16_t* v, int64_t 
                      bf16_t* dk, bf16_t* dv, int64_t lddv, int64_t N, int nq, int nkv, int B,
                      float scale, const int64_t* ds_base, int64_t ds_blocks, hipStream_t st);
 
+void fa128_few_launch(const bf16_t* q, const bf16_t* k, const bf16_t* v, int64_t ldv,
+                      const int64_t* bounds, const int32_t* tiles, int64_t n_tiles, bf16_t* o,
+                      float* lse, int64_t N, int nq, int nkv, int B, float scale, hipStream_t st);
 bool attn_f32_eligible(int64_t rows, int64_t nq, int64_t nkv, int64_t dh, int64_t ldv);
 void attn_f32_fwd_launch(const float* q, const float* k, const float* v, int64_t ldv,
                          const int64_t* bounds, const int32_t* row_segment, float* o, float* lse,
@@ -245,6 +249,10 @@ static bool use_mfma(int dtype, int64_t dh, const int32_t* tiles, int64_t ldv,
   return true;
 }
 
+// 128-row workgroups below which the forward takes 32-row ones whose waves
+// share the keys (attention_few.hip).
+constexpr int64_t FEW_WORKGROUPS = 256;
+
 extern "C" int alodlm_attention_fwd(const void* q, const void* k, const void* v, int64_t ldv,
                                     const int64_t* bounds, const int32_t* row_segment,
                                     const int32_t* tiles, int64_t n_tiles, void* o, float* lse,
@@ -257,6 +265,13 @@ extern "C" int alodlm_attention_fwd(const void* q, const void* k, const void* v,
   if (use_mfma(dtype, dh, tiles, ldv, {q, k, v, o})) {
     if (n_tiles == 0) return ALODLM_OK;
     ALODLM_CHECK_ARG(n_tiles <= 65535, "attention: too many 128-row tiles (%lld)", (long long)n_tiles);
+    if (dh == 128 && n_tiles * nq < FEW_WORKGROUPS && 4 * n_tiles <= 65535) {
+      fa128_few_launch((const bf16_t*)q, (const bf16_t*)k, (const bf16_t*)v, ldv, bounds, tiles,
+                       n_tiles, (bf16_t*)o, lse, rows, (int)nq, (int)nkv, (int)block_size, scale,
+                       as_stream(stream));
+      ALODLM_CHECK_LAUNCH("attention_fwd_few");
+      return ALODLM_OK;
+    }
     if (dh == 128)
       return fa128_fwd_launch((const bf16_t*)q, (const bf16_t*)k, (const bf16_t*)v, ldv, bounds,
                               tiles, n_tiles, (bf16_t*)o, lse, rows, (int)nq, (int)nkv,

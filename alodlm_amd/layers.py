@@ -185,17 +185,16 @@ class WindowMask:
     stream of one dual-stream segment of length P + W whose first P rows are
     the cache.
 
-    The MFMA kernels take 128-row query tiles from ``base`` = floor(P / 128) *
-    128, so the query buffer also holds rows [base, P) (zeros; their outputs
-    are ignored); the generic kernels take any row, so ``base`` = P there.
-    Segment row r is query-buffer row r - base and key/value row r (the
-    key/value pointers are offset by ``base`` rows)."""
+    Segment row r is query-buffer row r - P and key/value row r (the
+    key/value pointers are offset by ``base`` = P rows, so the cached keys lie
+    at negative rows); with ``tiled`` the MFMA kernels' query tiles start at
+    row P."""
 
     def __init__(self, prefix, window, tiled, device, block_size=1):
         self.prefix, self.window = prefix, window
         L = prefix + window
         self.block_size = block_size
-        self.base = (prefix // TILE_ROWS) * TILE_ROWS if tiled else prefix
+        self.base = prefix
         self.q_rows = L - self.base
         self.q_off = prefix - self.base
         self.boundaries = torch.tensor([-self.base, 2 * L - self.base], dtype=torch.int64,
