@@ -43,6 +43,8 @@ SIGNATURES = {
     "alodlm_qknorm_rope_fwd": [P, P, P, P, P, P, P, I64, I64, I64, I64, F32, I32, P],
     "alodlm_qknorm_rope_bwd_workspace": [I64, I64, I64, I64],
     "alodlm_qknorm_rope_bwd": [P, P, P, P, P, P, P, P, P, P, P, I64, I64, I64, I64, F32, I32, P],
+    "alodlm_norm_product": [P, I64, P, F32, P, I64, P, I64, I64, I64, I64, I32, I32, P],
+    "alodlm_qknorm_rotary_window": [P, P, P, P, P, P, P, P, I64, I64, I64, I64, F32, I32, P],
     "alodlm_qknorm_rotary_fwd": [P, P, P, P, P, P, P, I64, I64, I64, I64, F32, I32, P],
     "alodlm_qknorm_rotary_bwd": [P, P, P, P, P, P, P, P, P, P, P, I64, I64, I64, I64, F32, I32,
                                  P],

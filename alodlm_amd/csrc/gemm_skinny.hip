@@ -47,24 +47,47 @@ template <> struct SkinnyType<float> {
   }
 };
 
+// One 16-byte chunk of a bf16 row of x, normalised: w * cast(x * r), as the RMSNorm
+// kernels round.
+__device__ __forceinline__ uint4 normed(uint4 x, uint4 w, float r) {
+  const uint32_t xv[4] = {x.x, x.y, x.z, x.w}, wv[4] = {w.x, w.y, w.z, w.w};
+  uint32_t o[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const uint32_t t = pack_bf16x2(bf16_to_float((bf16_t)(xv[e] & 0xffffu)) * r,
+                                   bf16_to_float((bf16_t)(xv[e] >> 16)) * r);
+    o[e] = pack_bf16x2(bf16_to_float((bf16_t)(wv[e] & 0xffffu)) * bf16_to_float((bf16_t)(t & 0xffffu)),
+                       bf16_to_float((bf16_t)(wv[e] >> 16)) * bf16_to_float((bf16_t)(t >> 16)));
+  }
+  return make_uint4(o[0], o[1], o[2], o[3]);
+}
+// What the product does beside A W^T (bf16): SKINNY_NORM takes A through an
+// RMSNorm (weight nw, eps) first, SKINNY_GLU has W's first half of rows as gate and its
+// second half as up projection and stores silu(gate) * up (N / 2 columns).
+constexpr int SKINNY_NORM = 1, SKINNY_GLU = 2;
+
 // MT: 16-row blocks of A; NT: 16-row blocks of W per workgroup; U: fragment
 // pairs per operand block and register set (two sets: one loading, one used).
-template <typename T, int MT, int NT, int U, int EPI>
+template <typename T, int MT, int NT, int U, int EPI, int FUSE = 0>
 __global__ void __launch_bounds__(64 * WAVES)
 gemm_skinny_kernel(const T* __restrict__ A, int64_t lda, const T* __restrict__ W, int64_t ldw,
-                   T* C, int64_t ldc, const T* R, int64_t ldr, int M, int N, int K, float alpha) {
+                   T* C, int64_t ldc, const T* R, int64_t ldr, int M, int N, int K, float alpha,
+                   const T* __restrict__ nw, float eps) {
   typedef SkinnyType<T> S;
   constexpr int STEP = 2 * S::KS;  // k per fragment pair
   constexpr int COLS = 16 * NT, ROWS = 16 * MT;
+  constexpr bool NORM = FUSE & SKINNY_NORM, GLU = FUSE & SKINNY_GLU;
+  static_assert(!GLU || NT == 2, "one gate block and one up block");
   __shared__ __attribute__((aligned(16))) float red[WAVES][ROWS][COLS];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int i = lane & 15, kl = S::VEC * (lane >> 4);
-  const int n0 = blockIdx.x * COLS;
+  const int n0 = blockIdx.x * (GLU ? 16 : COLS);
+  const int cols = GLU ? N / 2 : N;  // of the output
   // Operands as buffers based at the workgroup's rows: one 32-bit lane offset
   // per block, and a chunk past K reads at an offset the range check turns
   // into zeros, so the loop has no branch around a load.
   constexpr uint32_t ES = sizeof(T), OUT = 0xffffff00u;
-  const int64_t nrows = N - n0 < COLS ? N - n0 : COLS;
+  const int64_t nrows = GLU ? N - n0 : N - n0 < COLS ? N - n0 : COLS;
   const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc(
       const_cast<T*>(W) + (int64_t)n0 * ldw, 0, (int)(((nrows - 1) * ldw + K) * ES), 0x00020000);
   const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc(
@@ -72,8 +95,9 @@ gemm_skinny_kernel(const T* __restrict__ A, int64_t lda, const T* __restrict__ W
   uint32_t wo[NT], xo[MT];
 #pragma unroll
   for (int b = 0; b < NT; ++b) {  // rows past the edge re-read the last one (never stored)
-    const int r = 16 * b + i;
-    wo[b] = (uint32_t)(((r < nrows ? r : nrows - 1) * ldw + kl) * ES);
+    const int64_t r = GLU ? (int64_t)b * cols + (n0 + i < cols ? i : cols - 1 - n0)
+                          : 16 * b + i < nrows ? 16 * b + i : nrows - 1;
+    wo[b] = (uint32_t)((r * ldw + kl) * ES);
   }
 #pragma unroll
   for (int a = 0; a < MT; ++a) {
@@ -86,7 +110,30 @@ gemm_skinny_kernel(const T* __restrict__ A, int64_t lda, const T* __restrict__ W
 #pragma unroll
     for (int b = 0; b < NT; ++b) acc[a][b] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 
-  uint4 w[2][U][2][NT], x[2][U][2][MT];
+  // 1 / rms of the rows (every workgroup for itself: 16 rows of 2048 are 64 KB
+  // from L2, less than a launch of its own costs)
+  float rs[MT];
+  __amdgpu_buffer_rsrc_t nr;
+  if constexpr (NORM) {
+    __shared__ float inv_rms[ROWS];
+    nr = __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(nw), 0, (int)(K * ES), 0x00020000);
+    for (int m = wave; m < M; m += WAVES) {
+      float s = 0.f;
+      for (int c = lane * 8; c < K; c += 512) {  // the RMSNorm kernels' order: the same bits
+        float v[8];
+        Vec8<T>::load(A + (int64_t)m * lda + c, v);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) s = fmaf(v[e], v[e], s);
+      }
+      s = wave_sum(s);
+      if (lane == 0) inv_rms[m] = 1.0f / sqrtf(s / (float)K + eps);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int a = 0; a < MT; ++a) rs[a] = inv_rms[16 * a + i < M ? 16 * a + i : M - 1];
+  }
+
+  uint4 w[2][U][2][NT], x[2][U][2][MT], nv[NORM ? 2 : 1][U][2];
   auto fetch = [&](const int set, const int k) {
 #pragma unroll
     for (int u = 0; u < U; ++u)
@@ -98,6 +145,9 @@ gemm_skinny_kernel(const T* __restrict__ A, int64_t lda, const T* __restrict__ W
         for (int b = 0; b < NT; ++b)
           w[set][u][h][b] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(
               wr, in ? wo[b] + kk * ES : OUT, 0, 0));
+        if constexpr (NORM)
+          nv[set][u][h] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(
+              nr, in ? (kk + kl) * ES : OUT, 0, 0));
 #pragma unroll
         for (int a = 0; a < MT; ++a)
           x[set][u][h][a] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(
@@ -110,10 +160,12 @@ gemm_skinny_kernel(const T* __restrict__ A, int64_t lda, const T* __restrict__ W
 #pragma unroll
       for (int h = 0; h < 2; ++h)
 #pragma unroll
-        for (int a = 0; a < MT; ++a)
+        for (int a = 0; a < MT; ++a) {
+          uint4 xa = x[set][u][h][a];
+          if constexpr (NORM) xa = normed(xa, nv[set][u][h], rs[a]);
 #pragma unroll
-          for (int b = 0; b < NT; ++b)
-            acc[a][b] = S::mma(w[set][u][h][b], x[set][u][h][a], acc[a][b]);
+          for (int b = 0; b < NT; ++b) acc[a][b] = S::mma(w[set][u][h][b], xa, acc[a][b]);
+        }
   };
   constexpr int SPAN = U * WAVES * STEP;
   const int k0 = wave * STEP;
@@ -134,13 +186,21 @@ gemm_skinny_kernel(const T* __restrict__ A, int64_t lda, const T* __restrict__ W
     for (int b = 0; b < NT; ++b)
       *reinterpret_cast<f32x4_t*>(&red[wave][16 * a + i][16 * b + 4 * (lane >> 4)]) = acc[a][b];
   __syncthreads();
-  for (int t = threadIdx.x; t < ROWS * COLS; t += 64 * WAVES) {
-    const int m = t / COLS, n = n0 + t % COLS;
-    if (m >= M || n >= N) continue;
+  constexpr int OUTS = GLU ? 16 : COLS;
+  for (int t = threadIdx.x; t < ROWS * OUTS; t += 64 * WAVES) {
+    const int m = t / OUTS, c = t % OUTS, n = n0 + c;
+    if (m >= M || n >= cols) continue;
     float v = 0.f;
 #pragma unroll
-    for (int s = 0; s < WAVES; ++s) v += red[s][m][t % COLS];
+    for (int s = 0; s < WAVES; ++s) v += red[s][m][c];
     v *= alpha;
+    if constexpr (GLU) {
+      float up = 0.f;
+#pragma unroll
+      for (int s = 0; s < WAVES; ++s) up += red[s][m][16 + c];
+      const float g = Elem<T>::round(v);
+      v = Elem<T>::round(g / (1.0f + expf(-g))) * Elem<T>::round(alpha * up);
+    }
     if (EPI == ALODLM_EPI_RESIDUAL) v = Elem<T>::load(R, m * ldr + n) + Elem<T>::round(v);
     Elem<T>::store(C, m * ldc + n, v);
   }
@@ -152,10 +212,10 @@ void launch(const T* A, int64_t lda, const T* W, int64_t ldw, T* C, int64_t ldc,
   const unsigned grid = ceil_div_u(N, 16 * NT);
   if (epi == ALODLM_EPI_STORE)
     gemm_skinny_kernel<T, MT, NT, U, ALODLM_EPI_STORE><<<grid, 64 * WAVES, 0, st>>>(
-        A, lda, W, ldw, C, ldc, R, ldr, M, N, K, alpha);
+        A, lda, W, ldw, C, ldc, R, ldr, M, N, K, alpha, nullptr, 0.f);
   else
     gemm_skinny_kernel<T, MT, NT, U, ALODLM_EPI_RESIDUAL><<<grid, 64 * WAVES, 0, st>>>(
-        A, lda, W, ldw, C, ldc, R, ldr, M, N, K, alpha);
+        A, lda, W, ldw, C, ldc, R, ldr, M, N, K, alpha, nullptr, 0.f);
 }
 
 template <typename T, int NT>
@@ -185,6 +245,24 @@ void launch_typed(const void* A, int64_t lda, const void* W, int64_t ldw, void* 
                       (int)N, (int)K, alpha, epi, st);
 }
 
+// 16 rows after 300 cached ones at the 1.7B shapes, a whole decoder layer call:
+// 92 us with the norms, the products, SwiGLU and the value copy in launches of
+// their own, 66 us with both norms and SwiGLU in the products and the values
+// copied by the rotary kernel.  float rows lose (154 us to 163): their norm
+// re-reads twice the bytes.
+void launch_fused(const bf16_t* A, int64_t lda, const bf16_t* nw, float eps, const bf16_t* W,
+                  int64_t ldw, bf16_t* C, int64_t ldc, int M, int N, int K, bool glu,
+                  hipStream_t st) {
+  if (glu)
+    gemm_skinny_kernel<bf16_t, 1, 2, 2, ALODLM_EPI_STORE, SKINNY_NORM | SKINNY_GLU>
+        <<<ceil_div_u(N / 2, 16), 64 * WAVES, 0, st>>>(A, lda, W, ldw, C, ldc, nullptr, 0, M, N, K,
+                                                       1.f, nw, eps);
+  else
+    gemm_skinny_kernel<bf16_t, 1, 1, 2, ALODLM_EPI_STORE, SKINNY_NORM>
+        <<<ceil_div_u(N, 16), 64 * WAVES, 0, st>>>(A, lda, W, ldw, C, ldc, nullptr, 0, M, N, K, 1.f,
+                                                   nw, eps);
+}
+
 }  // namespace
 
 bool gemm_skinny_eligible(const void* A, int64_t lda, int a_kmajor, const void* B, int64_t ldb,
@@ -206,4 +284,23 @@ void gemm_skinny_launch(const void* A, int64_t lda, const void* B, int64_t ldb, 
     launch_typed<bf16_t>(A, lda, B, ldb, C, ldc, R, ldr, M, N, K, alpha, epi, st);
   else
     launch_typed<float>(A, lda, B, ldb, C, ldc, R, ldr, M, N, K, alpha, epi, st);
+}
+
+// C = rmsnorm(x) W^T, or with `swiglu` silu(gate) * up of its two halves, for
+// at most 16 bf16 rows; returns ALODLM_EINVAL for anything wider or unaligned.
+extern "C" int alodlm_norm_product(const void* x, int64_t ldx, const void* norm_weight, float eps,
+                                   const void* W, int64_t ldw, void* C, int64_t ldc, int64_t M,
+                                   int64_t N, int64_t K, int swiglu, int dtype, void* stream) {
+  ALODLM_CHECK_ARG(dtype == ALODLM_BF16, "norm_product: bf16 only");
+  ALODLM_CHECK_ARG(M >= 0 && M <= 16, "norm_product: at most 16 rows");
+  if (M == 0 || N == 0) return ALODLM_OK;
+  ALODLM_CHECK_ARG(gemm_skinny_eligible(x, ldx, 1, W, ldw, 1, M, N, K, ALODLM_EPI_STORE, dtype) &&
+                       reinterpret_cast<uintptr_t>(norm_weight) % 16 == 0 &&
+                       N * ldw * 2 < (1LL << 31),
+                   "norm_product: rows must be 16-byte aligned and the weight below 2 GiB");
+  ALODLM_CHECK_ARG(!swiglu || N % 2 == 0, "norm_product: gate and up rows must pair");
+  launch_fused((const bf16_t*)x, ldx, (const bf16_t*)norm_weight, eps, (const bf16_t*)W, ldw,
+               (bf16_t*)C, ldc, (int)M, (int)N, (int)K, swiglu, as_stream(stream));
+  ALODLM_CHECK_LAUNCH("norm_product");
+  return ALODLM_OK;
 }

@@ -28,7 +28,9 @@ __device__ __forceinline__ void store_chunk(T* p, int64_t c, const float* v) {
 }
 
 // ---------------------------------------------------------------------------
-// y = w * cast(x * rsqrt(mean(x^2) + eps))
+// y = w * cast(x * rsqrt(mean(x^2) + eps)).  The squares are added by explicit
+// fused multiply-adds, so that the norm inside alodlm_norm_product gives the
+// same bits.
 // ---------------------------------------------------------------------------
 template <typename T, bool V8>
 __global__ void __launch_bounds__(64 * NORM_WAVES)
@@ -45,7 +47,7 @@ rmsnorm_fwd_kernel(const T* __restrict__ x, const T* __restrict__ w, T* __restri
     float v[8];
     load_chunk<T, V8>(xr, c, v);
 #pragma unroll
-    for (int i = 0; i < W; ++i) ss += v[i] * v[i];
+    for (int i = 0; i < W; ++i) ss = fmaf(v[i], v[i], ss);
   }
   ss = wave_sum(ss);
   const float r = 1.0f / sqrtf(ss / (float)cols + eps);
@@ -113,7 +115,7 @@ rmsnorm_fwd_vec_kernel(const T* __restrict__ x, const T* __restrict__ w, T* __re
           const uint32_t wd[4] = {cur[t].x, cur[t].y, cur[t].z, cur[t].w};
           Vec8<bf16_t>::unpack(wd, v[t]);
 #pragma unroll
-          for (int i = 0; i < 8; ++i) ss += v[t][i] * v[t][i];
+          for (int i = 0; i < 8; ++i) ss = fmaf(v[t][i], v[t][i], ss);
         }
       }
       ss = wave_sum(ss);
@@ -145,7 +147,7 @@ rmsnorm_fwd_vec_kernel(const T* __restrict__ x, const T* __restrict__ w, T* __re
       if (c < cols) {
         Vec8<T>::load(xr + c, v[t]);
 #pragma unroll
-        for (int i = 0; i < 8; ++i) ss += v[t][i] * v[t][i];
+        for (int i = 0; i < 8; ++i) ss = fmaf(v[t][i], v[t][i], ss);
       }
     }
     ss = wave_sum(ss);

@@ -41,8 +41,8 @@ __global__ void __launch_bounds__(64 * ROPE_WAVES)
 qknorm_rope_fwd_kernel(const T* __restrict__ qkv, const T* __restrict__ wq, const T* __restrict__ wk,
                        const int64_t* __restrict__ positions, const float* __restrict__ inv_freq,
                        const T* __restrict__ cos_tab, const T* __restrict__ sin_tab,
-                       T* __restrict__ q_out, T* __restrict__ k_out, int64_t rows, int nq, int nkv,
-                       int dh, float eps) {
+                       T* __restrict__ q_out, T* __restrict__ k_out, T* __restrict__ v_out,
+                       int64_t rows, int nq, int nkv, int dh, float eps) {
   const int lane = threadIdx.x & 63;
   const int64_t row = (int64_t)blockIdx.x * ROPE_WAVES + (threadIdx.x >> 6);
   if (row >= rows) return;
@@ -89,6 +89,8 @@ qknorm_rope_fwd_kernel(const T* __restrict__ qkv, const T* __restrict__ wq, cons
       }
     }
   }
+  if (v_out)  // the value heads as they are
+    for (int e = lane; e < nkv * dh; e += 64) v_out[row * nkv * dh + e] = src[(nq + nkv) * dh + e];
 }
 
 // Backward: dt = rotary^T d(out), then the RMSNorm backward over dh.  Per-lane
@@ -228,7 +230,8 @@ qknorm_rope128_fwd_kernel(const bf16_t* __restrict__ qkv, const bf16_t* __restri
                           const bf16_t* __restrict__ wk, const int64_t* __restrict__ positions,
                           const float* __restrict__ inv_freq, const bf16_t* __restrict__ cos_tab,
                           const bf16_t* __restrict__ sin_tab, bf16_t* __restrict__ q_out,
-                          bf16_t* __restrict__ k_out, int64_t rows, int nq, int nkv, float eps) {
+                          bf16_t* __restrict__ k_out, bf16_t* __restrict__ v_out, int64_t rows,
+                          int nq, int nkv, float eps) {
   const int lane = threadIdx.x & 63, slot = lane >> 3, j = lane & 7;
   const int64_t row = (int64_t)blockIdx.x * ROPE_WAVES + (threadIdx.x >> 6);
   if (row >= rows) return;
@@ -255,11 +258,20 @@ qknorm_rope128_fwd_kernel(const bf16_t* __restrict__ qkv, const bf16_t* __restri
   const float* sb = TAB ? sb_ : sn;
   Vec8<bf16_t>::load(wq + i0, wqa); Vec8<bf16_t>::load(wq + i0 + 64, wqb);
   Vec8<bf16_t>::load(wk + i0, wka); Vec8<bf16_t>::load(wk + i0 + 64, wkb);
-  const int heads = nq + nkv;
+  const int normed = nq + nkv, heads = v_out ? normed + nkv : normed;
   const bf16_t* src = qkv + row * (int64_t)(nq + 2 * nkv) * 128;
   for (int h0 = 8 * blockIdx.y; h0 < heads; h0 += 8 * gridDim.y) {
     const int head = h0 + slot;
-    const bool live = head < heads;
+    if (head >= normed) {  // a value head, as it is
+      if (head < heads) {
+        bf16_t* dst = v_out + (row * nkv + head - normed) * 128;
+        *reinterpret_cast<uint4*>(dst + i0) = *reinterpret_cast<const uint4*>(src + head * 128 + i0);
+        *reinterpret_cast<uint4*>(dst + i0 + 64) =
+            *reinterpret_cast<const uint4*>(src + head * 128 + i0 + 64);
+      }
+      continue;  // the head's 8 lanes together
+    }
+    const bool live = true;
     const bool is_q = head < nq;
     float xa[8], xb[8];
 #pragma unroll
@@ -397,8 +409,8 @@ static bool rope128_aligned16(const void* a, const void* b, const void* c) {
 // row's groups where the rows alone fill the chip (four wavefronts per SIMD),
 // else each group gets its own (a decoder window's 16 rows of 24 heads: three
 // short walks side by side instead of one of three).
-static dim3 rope128_grid(int64_t rows, int64_t nq, int64_t nkv) {
-  const unsigned groups = rows < 4096 ? ceil_div_u(nq + nkv, 8) : 1;
+static dim3 rope128_grid(int64_t rows, int64_t heads) {
+  const unsigned groups = rows < 4096 ? ceil_div_u(heads, 8) : 1;
   return dim3(ceil_div_u(rows, ROPE_WAVES), groups < 65535 ? groups : 65535);
 }
 
@@ -419,16 +431,16 @@ extern "C" int alodlm_qknorm_rope_fwd(const void* qkv, const void* wq, const voi
   ALODLM_DISPATCH(dtype, T, {
     if (std::is_same<T, bf16_t>::value && dh == 128 && rope128_aligned16(qkv, q_out, k_out) &&
         rope128_aligned16(wq, wk, wk)) {
-      qknorm_rope128_fwd_kernel<false><<<rope128_grid(rows, nq, nkv), 64 * ROPE_WAVES, 0,
+      qknorm_rope128_fwd_kernel<false><<<rope128_grid(rows, nq + nkv), 64 * ROPE_WAVES, 0,
                                          as_stream(stream)>>>(
           (const bf16_t*)qkv, (const bf16_t*)wq, (const bf16_t*)wk, positions, inv_freq, nullptr,
-          nullptr, (bf16_t*)q_out, (bf16_t*)k_out, rows, (int)nq, (int)nkv, eps);
+          nullptr, (bf16_t*)q_out, (bf16_t*)k_out, nullptr, rows, (int)nq, (int)nkv, eps);
       break;
     }
     qknorm_rope_fwd_kernel<T, false><<<ceil_div_u(rows, ROPE_WAVES), 64 * ROPE_WAVES, 0,
                                        as_stream(stream)>>>(
         (const T*)qkv, (const T*)wq, (const T*)wk, positions, inv_freq, nullptr, nullptr,
-        (T*)q_out, (T*)k_out, rows, (int)nq, (int)nkv, (int)dh, eps);
+        (T*)q_out, (T*)k_out, nullptr, rows, (int)nq, (int)nkv, (int)dh, eps);
   });
   ALODLM_CHECK_LAUNCH("qknorm_rope_fwd");
   return ALODLM_OK;
@@ -488,30 +500,47 @@ extern "C" int alodlm_qknorm_rope_bwd(const void* dq, const void* dk, const void
 // Table-driven forms (alodlm/model.py:41-46 takes cos/sin tables [rows, dh]):
 // q/k norm + rotary on the projections, and the rotary alone.
 // ---------------------------------------------------------------------------
-extern "C" int alodlm_qknorm_rotary_fwd(const void* qkv, const void* wq, const void* wk,
-                                        const void* cos_tab, const void* sin_tab, void* q_out,
-                                        void* k_out, int64_t rows, int64_t nq, int64_t nkv,
-                                        int64_t dh, float eps, int dtype, void* stream) {
+// v_out (or null) receives the value heads unchanged, [rows, nkv * dh].
+static int rotary_fwd_launch(const void* qkv, const void* wq, const void* wk, const void* cos_tab,
+                             const void* sin_tab, void* q_out, void* k_out, void* v_out,
+                             int64_t rows, int64_t nq, int64_t nkv, int64_t dh, float eps,
+                             int dtype, hipStream_t st) {
   int rc = check_rope(rows, nq, nkv, dh);
   if (rc) return rc;
   if (rows == 0) return ALODLM_OK;
   ALODLM_DISPATCH(dtype, T, {
     if (std::is_same<T, bf16_t>::value && dh == 128 && rope128_aligned16(qkv, q_out, k_out) &&
-        rope128_aligned16(wq, wk, wk) && rope128_aligned16(cos_tab, sin_tab, sin_tab)) {
-      qknorm_rope128_fwd_kernel<true><<<rope128_grid(rows, nq, nkv), 64 * ROPE_WAVES, 0,
-                                        as_stream(stream)>>>(
+        rope128_aligned16(wq, wk, v_out) && rope128_aligned16(cos_tab, sin_tab, sin_tab)) {
+      qknorm_rope128_fwd_kernel<true><<<rope128_grid(rows, nq + nkv + (v_out ? nkv : 0)),
+                                        64 * ROPE_WAVES, 0, st>>>(
           (const bf16_t*)qkv, (const bf16_t*)wq, (const bf16_t*)wk, nullptr, nullptr,
-          (const bf16_t*)cos_tab, (const bf16_t*)sin_tab, (bf16_t*)q_out, (bf16_t*)k_out, rows,
-          (int)nq, (int)nkv, eps);
+          (const bf16_t*)cos_tab, (const bf16_t*)sin_tab, (bf16_t*)q_out, (bf16_t*)k_out,
+          (bf16_t*)v_out, rows, (int)nq, (int)nkv, eps);
       break;
     }
-    qknorm_rope_fwd_kernel<T, true><<<ceil_div_u(rows, ROPE_WAVES), 64 * ROPE_WAVES, 0,
-                                      as_stream(stream)>>>(
+    qknorm_rope_fwd_kernel<T, true><<<ceil_div_u(rows, ROPE_WAVES), 64 * ROPE_WAVES, 0, st>>>(
         (const T*)qkv, (const T*)wq, (const T*)wk, nullptr, nullptr, (const T*)cos_tab,
-        (const T*)sin_tab, (T*)q_out, (T*)k_out, rows, (int)nq, (int)nkv, (int)dh, eps);
+        (const T*)sin_tab, (T*)q_out, (T*)k_out, (T*)v_out, rows, (int)nq, (int)nkv, (int)dh, eps);
   });
   ALODLM_CHECK_LAUNCH("qknorm_rotary_fwd");
   return ALODLM_OK;
+}
+
+extern "C" int alodlm_qknorm_rotary_fwd(const void* qkv, const void* wq, const void* wk,
+                                        const void* cos_tab, const void* sin_tab, void* q_out,
+                                        void* k_out, int64_t rows, int64_t nq, int64_t nkv,
+                                        int64_t dh, float eps, int dtype, void* stream) {
+  return rotary_fwd_launch(qkv, wq, wk, cos_tab, sin_tab, q_out, k_out, nullptr, rows, nq, nkv, dh,
+                           eps, dtype, as_stream(stream));
+}
+
+extern "C" int alodlm_qknorm_rotary_window(const void* qkv, const void* wq, const void* wk,
+                                           const void* cos_tab, const void* sin_tab, void* q_out,
+                                           void* k_out, void* v_out, int64_t rows, int64_t nq,
+                                           int64_t nkv, int64_t dh, float eps, int dtype,
+                                           void* stream) {
+  return rotary_fwd_launch(qkv, wq, wk, cos_tab, sin_tab, q_out, k_out, v_out, rows, nq, nkv, dh,
+                           eps, dtype, as_stream(stream));
 }
 
 extern "C" int alodlm_qknorm_rotary_bwd(const void* dq, const void* dk, const void* qkv,

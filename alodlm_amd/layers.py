@@ -32,6 +32,7 @@ from ._lib import EPI_ACCUM, EPI_RESIDUAL, EPI_STORE, EPI_STORE_F32, call, ptr, 
 
 TILE_ROWS = 128
 SKINNY_ROWS = 64  # rows up to which a product streams its [out, in] weight
+FUSED_ROWS = 16  # bf16 rows up to which norm, product and SwiGLU are one launch
 
 
 def allowed_pairs(length, block_size):
@@ -340,6 +341,27 @@ class Kernels:
         else:
             self._gemm(x, ldx, 1, w, K, 1, y, N, M, N, K, epi=epi, R=R, ldr=ldr)
 
+    def _norm_product(self, x, norm, w, w_t, N, swiglu=False):
+        """rmsnorm(x) . w^T over a window's rows x [M, K], w [N, K]; with
+        ``swiglu`` silu(gate) * up of its two halves.  Up to FUSED_ROWS bf16
+        rows in one launch, else one per step."""
+        d, st, c = self.dims, self._stream(), self.code
+        M, K = x.shape
+        out = self._empty(M, N // 2 if swiglu else N)
+        if (M <= FUSED_ROWS and self.dtype == torch.bfloat16 and K % 8 == 0
+                and ptr(x) % 16 == 0 and ptr(norm) % 16 == 0
+                and ptr(w) % 16 == 0 and w.numel() * w.element_size() < 2 ** 31):
+            call("alodlm_norm_product", ptr(x), K, ptr(norm), d.eps, ptr(w), K, ptr(out),
+                 out.shape[1], M, N, K, int(swiglu), c, st)
+            return out
+        h = self._empty(M, K)
+        call("alodlm_rmsnorm_fwd", ptr(x), ptr(norm), ptr(h), None, M, K, d.eps, c, st)
+        y = self._empty(M, N) if swiglu else out
+        self._product(h, K, w, w_t, y, M, N, K)
+        if swiglu:
+            call("alodlm_swiglu_fwd", ptr(y), ptr(out), M, N // 2, c, st)
+        return out
+
     def _attention_fwd(self, q, k, v, ldv, o, lse, mask):
         d = self.dims
         call("alodlm_attention_fwd", ptr(q), ptr(k), ptr(v), ldv, ptr(mask.boundaries),
@@ -517,33 +539,23 @@ class Kernels:
         H, QW, I = d.hidden, d.qkv_width, d.intermediate
         QD, KD = d.heads * d.head_dim, d.kv_heads * d.head_dim
         esize = x.element_size()
-        h1 = self._empty(Wn, H)
-        call("alodlm_rmsnorm_fwd", ptr(x), ptr(w.ln1), ptr(h1), None, Wn, H, d.eps, c, st)
-        qkv = self._empty(Wn, QW)
-        self._product(h1, H, w.wqkv, w.wqkv_t, qkv, Wn, QW, H)
-        q_all = self._empty(mask.q_rows, QD)
-        if mask.q_off:
-            q_all[:mask.q_off].zero_()
-        q_view = q_all[mask.q_off:]
+        qkv = self._norm_product(x, w.ln1, w.wqkv, w.wqkv_t, QW)
+        q = self._empty(Wn, QD)
         k_view = kbuf.view(-1, KD)[mask.prefix:mask.prefix + Wn]
-        self._rope_fwd(qkv, w, rope, q_view, k_view)
-        vbuf.view(-1, KD)[mask.prefix:mask.prefix + Wn].copy_(qkv[:, QD + KD:])
-        o_all = self._empty(mask.q_rows, QD)
-        lse = self._empty(d.heads, mask.q_rows, dtype=torch.float32)
+        v_view = vbuf.view(-1, KD)[mask.prefix:mask.prefix + Wn]
+        call("alodlm_qknorm_rotary_window", ptr(qkv), ptr(w.qn), ptr(w.kn), ptr(rope.cos),
+             ptr(rope.sin), ptr(q), ptr(k_view), ptr(v_view), Wn, d.heads,
+             d.kv_heads, d.head_dim, d.eps, c, st)
+        o = self._empty(Wn, QD)
+        lse = self._empty(d.heads, Wn, dtype=torch.float32)
         shift = mask.base * KD * esize
-        call("alodlm_attention_fwd", ptr(q_all), ptr(kbuf) + shift, ptr(vbuf) + shift, KD,
+        call("alodlm_attention_fwd", ptr(q), ptr(kbuf) + shift, ptr(vbuf) + shift, KD,
              ptr(mask.boundaries), ptr(mask.row_segment), ptr(mask.tiles),
-             0 if mask.tiles is None else mask.tiles.shape[0], ptr(o_all), ptr(lse), mask.q_rows,
+             0 if mask.tiles is None else mask.tiles.shape[0], ptr(o), ptr(lse), Wn,
              d.heads, d.kv_heads, d.head_dim, mask.block_size, c, st)
-        o = o_all[mask.q_off:]
         x1 = self._empty(Wn, H)
         self._product(o, QD, w.wo, w.wo_t, x1, Wn, H, QD, epi=EPI_RESIDUAL, R=x, ldr=H)
-        h2 = self._empty(Wn, H)
-        call("alodlm_rmsnorm_fwd", ptr(x1), ptr(w.ln2), ptr(h2), None, Wn, H, d.eps, c, st)
-        gu = self._empty(Wn, 2 * I)
-        self._product(h2, H, w.wgu, w.wgu_t, gu, Wn, 2 * I, H)
-        act = self._empty(Wn, I)
-        call("alodlm_swiglu_fwd", ptr(gu), ptr(act), Wn, I, c, st)
+        act = self._norm_product(x1, w.ln2, w.wgu, w.wgu_t, 2 * I, swiglu=True)
         y = self._empty(Wn, H)
         self._product(act, I, w.wd, w.wd_t, y, Wn, H, I, epi=EPI_RESIDUAL, R=x1, ldr=H)
         return y

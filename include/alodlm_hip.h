@@ -170,6 +170,12 @@ int alodlm_qknorm_rotary_fwd(const void* qkv, const void* wq, const void* wk, co
                              const void* sin_tab, void* q_out, void* k_out, int64_t rows,
                              int64_t nq, int64_t nkv, int64_t dh, float eps, int dtype,
                              void* stream);
+/* alodlm_qknorm_rotary_fwd that also writes the value heads unchanged to v_out
+ * [rows, nkv*dh] (a decoding window's place in the key/value cache). */
+int alodlm_qknorm_rotary_window(const void* qkv, const void* wq, const void* wk,
+                                const void* cos_tab, const void* sin_tab, void* q_out,
+                                void* k_out, void* v_out, int64_t rows, int64_t nq, int64_t nkv,
+                                int64_t dh, float eps, int dtype, void* stream);
 int alodlm_qknorm_rotary_bwd(const void* dq, const void* dk, const void* qkv, const void* wq,
                              const void* wk, const void* cos_tab, const void* sin_tab, void* dqkv,
                              float* dwq_accum, float* dwk_accum, float* workspace, int64_t rows,
@@ -209,6 +215,14 @@ int alodlm_gemm(const void* A, int64_t lda, int a_kmajor, const void* B, int64_t
                 int b_kmajor, void* C, int64_t ldc, const void* R, int64_t ldr, int64_t M,
                 int64_t N, int64_t K, float alpha, int epilogue, int dtype, float* workspace,
                 void* stream);
+/* C = rmsnorm(x) . W^T for at most 16 bf16 rows (alodlm/model.py:56-58,75 in a
+ * decoding window): x [M, K] of row stride ldx, W [N, K]; with `swiglu` W's rows
+ * are the gate then the up projection and C [M, N/2] = silu(gate) * up.  Each
+ * step rounds to dtype where the separate entry points do. */
+int alodlm_norm_product(const void* x, int64_t ldx, const void* norm_weight, float eps,
+                        const void* W, int64_t ldw, void* C, int64_t ldc, int64_t M, int64_t N,
+                        int64_t K, int swiglu, int dtype, void* stream);
+
 /* The weight gradient of a layer applied once per recurrent pass
  * (alodlm/model.py:152, the loop over depths, whose autograd sums the passes'
  * nn.Linear weight gradients) as one product:
