@@ -34,6 +34,14 @@ SIGNATURES = {
     "alodlm_embed_scatter": [P, P, P, I64, P, P, I64, I64, I64, I32, P],
     "alodlm_embed_scatter_add": [P, P, P, I64, P, P, I64, I64, I64, I32, P],
     "alodlm_rmsnorm_fwd": [P, P, P, P, I64, I64, F32, I32, P],
+    "alodlm_window_layer_scratch": [I64] * 6 + [I32],
+    "alodlm_window_layer": [P] * 17 + [I64, I64, P, P, P, I64, I64, P, P] + [I64] * 6
+                           + [F32, I32, P],
+    "alodlm_layer_saved": [I64] * 6 + [I32],
+    "alodlm_layer_fwd_scratch": [I64] * 6 + [I32],
+    "alodlm_layer_fwd": [P] * 16 + [I64, I64] + [P] * 5 + [I64] * 6 + [F32, I32, P],
+    "alodlm_layer_bwd_scratch": [I64] * 8 + [I32],
+    "alodlm_layer_bwd": [P] * 19 + [I64, P, I64, I64] + [P] * 10 + [I64] * 6 + [F32, I32, P],
     "alodlm_rmsnorm_bwd_workspace": [I64, I64],
     "alodlm_embed_plan_size": [I64],
     "alodlm_embed_scatter_workspace": [I64, I64],
@@ -97,6 +105,10 @@ SIGNATURES = {
 }
 _RESTYPE = {
     "alodlm_last_error": ctypes.c_char_p,
+    "alodlm_window_layer_scratch": I64,
+    "alodlm_layer_saved": I64,
+    "alodlm_layer_fwd_scratch": I64,
+    "alodlm_layer_bwd_scratch": I64,
     "alodlm_rmsnorm_bwd_workspace": I64,
     "alodlm_embed_plan_size": I64,
     "alodlm_embed_scatter_workspace": I64,

@@ -248,7 +248,7 @@ void launch_typed(const void* A, int64_t lda, const void* W, int64_t ldw, void* 
 // 16 rows after 300 cached ones at the 1.7B shapes, a whole decoder layer call:
 // 92 us with the norms, the products, SwiGLU and the value copy in launches of
 // their own, 66 us with both norms and SwiGLU in the products and the values
-// copied by the rotary kernel.  float rows lose (154 us to 163): their norm
+// copied by the rotary kernel.  float rows lose (154 us to 169): their norm
 // re-reads twice the bytes.
 void launch_fused(const bf16_t* A, int64_t lda, const bf16_t* nw, float eps, const bf16_t* W,
                   int64_t ldw, bf16_t* C, int64_t ldc, int M, int N, int K, bool glu,

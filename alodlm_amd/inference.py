@@ -28,11 +28,11 @@ How this implementation is organised:
   not a copy.
 * **Layers on the step's kernels.**  Every layer application is a call of
   the module-level ``layer_forward`` (``alodlm_amd.model``, bound here as the
-  reference binds it), which runs ``Kernels.layer_window``: RMSNorm, the
-  GEMMs, q/k-norm + RoPE, attention, SwiGLU, with the window's keys and
-  values written in place (``layers.WindowSlot``).  The window's mask (every cached key, causal inside the window;
-  alodlm/inference.py:77-79) is the clean stream of one dual-stream segment
-  (``WindowMask``).  The carry norm plus re-embedding is one ``carry_select``
+  reference binds it), which runs ``Kernels.layer_window``, one host call for
+  the layer's launches, with the window's keys and values written in place
+  (``layers.WindowSlot``).  The window's mask (every cached key, causal inside
+  the window; alodlm/inference.py:77-79) is the clean stream of one dual-stream
+  segment (``WindowMask``).  The carry norm plus re-embedding is one ``carry_select``
   launch, the final norm and gate one ``final_norm_gate`` launch, and the
   readout's argmax and entropy one ``decode_readout`` launch.
 """

@@ -1,11 +1,13 @@
 """One Qwen3 decoder layer on the HIP kernels.
 
-The forward and backward schedules of a layer application live here
-(``Kernels.layer_fwd``, ``layer_bwd``, ``layer_window``) and are shared by the
-fused training step (``engine.StepEngine``), the decoder and the reference's
-public layer functions, which ``alodlm_amd.model`` defines where the
-reference does (alodlm/model.py:41-80): ``rotary``, ``layer_forward`` and
-``training_layer`` run on the autograd nodes and mask forms of this module.
+``Kernels.layer_fwd`` and ``layer_bwd`` are the schedules of the fused training
+step (``engine.StepEngine``), which decides what a layer keeps and when its
+weight gradients run.  ``layer_call_fwd``, ``layer_call_bwd`` and
+``layer_window`` are single host calls for a layer by itself: the decoder's
+windows, the rollout, and the reference's public layer functions, which
+``alodlm_amd.model`` defines where the reference does (alodlm/model.py:41-80;
+``rotary``, ``layer_forward`` and ``training_layer`` run on the autograd nodes
+and mask forms of this module).
 
 The attention mask is one of
 
@@ -32,7 +34,6 @@ from ._lib import EPI_ACCUM, EPI_RESIDUAL, EPI_STORE, EPI_STORE_F32, call, ptr, 
 
 TILE_ROWS = 128
 SKINNY_ROWS = 64  # rows up to which a product streams its [out, in] weight
-FUSED_ROWS = 16  # bf16 rows up to which norm, product and SwiGLU are one launch
 
 
 def allowed_pairs(length, block_size):
@@ -341,27 +342,6 @@ class Kernels:
         else:
             self._gemm(x, ldx, 1, w, K, 1, y, N, M, N, K, epi=epi, R=R, ldr=ldr)
 
-    def _norm_product(self, x, norm, w, w_t, N, swiglu=False):
-        """rmsnorm(x) . w^T over a window's rows x [M, K], w [N, K]; with
-        ``swiglu`` silu(gate) * up of its two halves.  Up to FUSED_ROWS bf16
-        rows in one launch, else one per step."""
-        d, st, c = self.dims, self._stream(), self.code
-        M, K = x.shape
-        out = self._empty(M, N // 2 if swiglu else N)
-        if (M <= FUSED_ROWS and self.dtype == torch.bfloat16 and K % 8 == 0
-                and ptr(x) % 16 == 0 and ptr(norm) % 16 == 0
-                and ptr(w) % 16 == 0 and w.numel() * w.element_size() < 2 ** 31):
-            call("alodlm_norm_product", ptr(x), K, ptr(norm), d.eps, ptr(w), K, ptr(out),
-                 out.shape[1], M, N, K, int(swiglu), c, st)
-            return out
-        h = self._empty(M, K)
-        call("alodlm_rmsnorm_fwd", ptr(x), ptr(norm), ptr(h), None, M, K, d.eps, c, st)
-        y = self._empty(M, N) if swiglu else out
-        self._product(h, K, w, w_t, y, M, N, K)
-        if swiglu:
-            call("alodlm_swiglu_fwd", ptr(y), ptr(out), M, N // 2, c, st)
-        return out
-
     def _attention_fwd(self, q, k, v, ldv, o, lse, mask):
         d = self.dims
         call("alodlm_attention_fwd", ptr(q), ptr(k), ptr(v), ldv, ptr(mask.boundaries),
@@ -534,31 +514,58 @@ class Kernels:
         window's rotated keys and values are written into rows [P, P + W) of
         the key/value buffers kbuf/vbuf [capacity, kv_heads * head_dim], whose
         rows [0, P) hold the prefix; ``mask`` is a WindowMask."""
-        d, st, c = self.dims, self._stream(), self.code
-        Wn = x.shape[0]
-        H, QW, I = d.hidden, d.qkv_width, d.intermediate
-        QD, KD = d.heads * d.head_dim, d.kv_heads * d.head_dim
-        esize = x.element_size()
-        qkv = self._norm_product(x, w.ln1, w.wqkv, w.wqkv_t, QW)
-        q = self._empty(Wn, QD)
-        k_view = kbuf.view(-1, KD)[mask.prefix:mask.prefix + Wn]
-        v_view = vbuf.view(-1, KD)[mask.prefix:mask.prefix + Wn]
-        call("alodlm_qknorm_rotary_window", ptr(qkv), ptr(w.qn), ptr(w.kn), ptr(rope.cos),
-             ptr(rope.sin), ptr(q), ptr(k_view), ptr(v_view), Wn, d.heads,
-             d.kv_heads, d.head_dim, d.eps, c, st)
-        o = self._empty(Wn, QD)
-        lse = self._empty(d.heads, Wn, dtype=torch.float32)
-        shift = mask.base * KD * esize
-        call("alodlm_attention_fwd", ptr(q), ptr(kbuf) + shift, ptr(vbuf) + shift, KD,
+        rows, dims = x.shape[0], self._layer_dims(x.shape[0])
+        scratch = self._bytes("alodlm_window_layer_scratch", *dims, self.code)
+        y = self._empty(rows, self.dims.hidden)
+        call("alodlm_window_layer", ptr(x), ptr(w.wqkv), ptr(w.wqkv_t), ptr(w.wo), ptr(w.wo_t),
+             ptr(w.wgu), ptr(w.wgu_t), ptr(w.wd), ptr(w.wd_t), ptr(w.ln1), ptr(w.ln2), ptr(w.qn),
+             ptr(w.kn), ptr(rope.cos), ptr(rope.sin), ptr(kbuf), ptr(vbuf), mask.prefix, mask.base,
              ptr(mask.boundaries), ptr(mask.row_segment), ptr(mask.tiles),
-             0 if mask.tiles is None else mask.tiles.shape[0], ptr(o), ptr(lse), Wn,
-             d.heads, d.kv_heads, d.head_dim, mask.block_size, c, st)
-        x1 = self._empty(Wn, H)
-        self._product(o, QD, w.wo, w.wo_t, x1, Wn, H, QD, epi=EPI_RESIDUAL, R=x, ldr=H)
-        act = self._norm_product(x1, w.ln2, w.wgu, w.wgu_t, 2 * I, swiglu=True)
-        y = self._empty(Wn, H)
-        self._product(act, I, w.wd, w.wd_t, y, Wn, H, I, epi=EPI_RESIDUAL, R=x1, ldr=H)
+             0 if mask.tiles is None else mask.tiles.shape[0], mask.block_size, ptr(scratch),
+             ptr(y), *dims, self.dims.eps, self.code, self._stream())
         return y
+
+    def _layer_dims(self, rows):
+        d = self.dims
+        return rows, d.hidden, d.heads, d.kv_heads, d.head_dim, d.intermediate
+
+    def _bytes(self, size, *args):
+        return torch.empty(query(size, *args), dtype=torch.uint8, device=self.device)
+
+    def layer_call_fwd(self, w, x, rope, mask):
+        """One differentiable layer call over x [N, H] as one host call
+        (``layer_fwd``'s steps): returns y, the rotated keys, the values (None
+        without rotary tables) and the bytes ``layer_call_bwd`` reads."""
+        d, N = self.dims, x.shape[0]
+        dims = self._layer_dims(N)
+        saved = self._bytes("alodlm_layer_saved", *dims, self.code)
+        scratch = self._bytes("alodlm_layer_fwd_scratch", *dims, self.code)
+        k = self._empty(N, d.kv_heads, d.head_dim)
+        v = self._empty(N, d.kv_heads, d.head_dim) if rope.tables else None
+        y = self._empty(N, d.hidden)
+        call("alodlm_layer_fwd", ptr(x), ptr(w.wqkv), ptr(w.wo), ptr(w.wgu), ptr(w.wd), ptr(w.ln1),
+             ptr(w.ln2), ptr(w.qn), ptr(w.kn), ptr(rope.cos), ptr(rope.sin), ptr(rope.positions),
+             ptr(rope.inv_freq), ptr(mask.boundaries), ptr(mask.row_segment), ptr(mask.tiles),
+             0 if mask.tiles is None else mask.tiles.shape[0], mask.block_size, ptr(k), ptr(v),
+             ptr(saved), ptr(scratch), ptr(y), *dims, d.eps, self.code, self._stream())
+        return y, k, v, saved
+
+    def layer_call_bwd(self, dy, x, k, saved, w, gw, rope, mask):
+        """Backward of ``layer_call_fwd``: returns dx, writes the matrices'
+        gradients (``gw.stored``) and adds the norm weights' to ``gw``."""
+        d, dims = self.dims, self._layer_dims(x.shape[0])
+        n_tiles = 0 if mask.tiles is None else mask.tiles.shape[0]
+        ds_blocks = getattr(mask, "ds_blocks", 0)
+        scratch = self._bytes("alodlm_layer_bwd_scratch", *dims, n_tiles, ds_blocks, self.code)
+        dx = self._empty(*x.shape)
+        call("alodlm_layer_bwd", ptr(dy), ptr(x), ptr(k), ptr(saved), ptr(w.wqkv), ptr(w.wo),
+             ptr(w.wgu), ptr(w.wd), ptr(w.ln1), ptr(w.ln2), ptr(w.qn), ptr(w.kn), ptr(rope.cos),
+             ptr(rope.sin), ptr(rope.positions), ptr(rope.inv_freq), ptr(mask.boundaries),
+             ptr(mask.row_segment), ptr(mask.tiles), n_tiles,
+             ptr(getattr(mask, "ds_base", None)), ds_blocks, mask.block_size, ptr(gw.wqkv),
+             ptr(gw.wo), ptr(gw.wgu), ptr(gw.wd), ptr(gw.ln1), ptr(gw.ln2), ptr(gw.qn), ptr(gw.kn),
+             ptr(scratch), ptr(dx), *dims, d.eps, self.code, self._stream())
+        return dx
 
 
 # ----------------------------------------------------------------------------
@@ -615,18 +622,14 @@ class _LayerFunction(torch.autograd.Function):
     @staticmethod
     def forward(ctx, kernels, mask, rope, hidden, *params):
         w = LayerWeights.from_tensors(*params)
-        save = []
-        y = kernels.layer_fwd(w, hidden.contiguous(), mask, rope, save, keep=(True, False))
-        ctx.kernels, ctx.mask, ctx.rope, ctx.saved, ctx.w = kernels, mask, rope, save[0], w
+        x = hidden.contiguous()
+        y, k, v, saved = kernels.layer_call_fwd(w, x, rope, mask)
+        ctx.kernels, ctx.mask, ctx.rope, ctx.saved, ctx.w = kernels, mask, rope, (x, k, saved), w
         ctx.shapes = [(p.shape, p.dtype) for p in params]
-        d = kernels.dims
-        q, k = save[0][9], save[0][10]
-        qkv = save[0][3]
-        v = qkv[:, (d.heads + d.kv_heads) * d.head_dim:]
-        k_out = k.view(-1, d.kv_heads, d.head_dim)
-        v_out = v.contiguous().view(-1, d.kv_heads, d.head_dim)
-        ctx.mark_non_differentiable(k_out, v_out)
-        return y, k_out, v_out
+        if v is None:  # only a table-driven call hands its keys and values out
+            return y, None, None
+        ctx.mark_non_differentiable(k, v)
+        return y, k, v
 
     @staticmethod
     def backward(ctx, dy, _dk, _dv):
@@ -639,11 +642,14 @@ class _LayerFunction(torch.autograd.Function):
         gw = LayerGrads(mats[0].view(W, H), mats[1].view(H, QD), mats[2].view(2 * I, H),
                         mats[3].view(H, I), *norms.split([H, H, d.head_dim, d.head_dim]),
                         stored=True)
-        dx = kernels.layer_bwd(dy.contiguous(), ctx.saved, w, gw, ctx.mask, ctx.rope)
+        x, k, saved = ctx.saved
+        dx = kernels.layer_call_bwd(dy.contiguous(), x, k, saved, w, gw, ctx.rope, ctx.mask)
         ctx.saved = None
+        if len({dtype for _, dtype in ctx.shapes[7:]}) == 1:  # one cast for the four
+            norms = norms.to(ctx.shapes[7][1])
         qd, kd = QD, d.kv_heads * d.head_dim
         parts = [gw.wqkv[:qd], gw.wqkv[qd:qd + kd], gw.wqkv[qd + kd:], gw.wo, gw.wgu[:I],
-                 gw.wgu[I:], gw.wd, gw.ln1, gw.ln2, gw.qn, gw.kn]
+                 gw.wgu[I:], gw.wd, *norms.split([H, H, d.head_dim, d.head_dim])]
         grads = [g.view(shape).to(dtype) for g, (shape, dtype) in zip(parts, ctx.shapes)]
         return (None, None, None, dx, *grads)
 

@@ -223,6 +223,60 @@ int alodlm_norm_product(const void* x, int64_t ldx, const void* norm_weight, flo
                         const void* W, int64_t ldw, void* C, int64_t ldc, int64_t M, int64_t N,
                         int64_t K, int swiglu, int dtype, void* stream);
 
+/* One decoder layer over a decoding window (alodlm/inference.py:83-88): rows x
+ * [rows, hidden] after `prefix` cached rows, whose rotated keys and values are
+ * written into rows [prefix, prefix + rows) of kbuf / vbuf [.., nkv*dh]; y
+ * [rows, hidden].  Weights as alodlm_gemm takes them: w* [out, in], w*_t their
+ * [in, out] copies or NULL; cos/sin [rows, dh].  The attention's mask
+ * arguments are alodlm_attention_fwd's, its key rows start `base` rows into
+ * the buffers.  scratch: alodlm_window_layer_scratch(...) bytes, 256-byte
+ * aligned. */
+int64_t alodlm_window_layer_scratch(int64_t rows, int64_t hidden, int64_t nq, int64_t nkv,
+                                    int64_t dh, int64_t inter, int dtype);
+int alodlm_window_layer(
+    const void* x, const void* wqkv, const void* wqkv_t, const void* wo, const void* wo_t,
+    const void* wgu, const void* wgu_t, const void* wd, const void* wd_t, const void* ln1,
+    const void* ln2, const void* qn, const void* kn, const void* cos_tab, const void* sin_tab,
+    void* kbuf, void* vbuf, int64_t prefix, int64_t base, const int64_t* bounds,
+    const int32_t* row_segment, const int32_t* tiles, int64_t n_tiles, int64_t block_size,
+    void* scratch, void* y, int64_t rows, int64_t hidden, int64_t nq, int64_t nkv, int64_t dh,
+    int64_t inter, float eps, int dtype, void* stream);
+
+/* One differentiable decoder layer call (alodlm/model.py:49-76) as one host
+ * call each way, with the mask arguments of alodlm_attention_fwd / _bwd.
+ * Rotary tables cos/sin [rows, dh], or (both NULL) positions and inv_freq as
+ * alodlm_qknorm_rope_fwd takes them.  Forward: x -> y [rows, hidden], the
+ * rotated keys k and, with tables only (else v is NULL), the values v, both
+ * [rows, nkv*dh], and what the backward reads in `saved`
+ * (alodlm_layer_saved(...) bytes).  Backward: dx, the matrices' gradients in
+ * the storage dtype (written), the norm weights' in float32 (added).
+ * scratch: alodlm_layer_fwd_scratch(...) and _bwd_scratch(...) bytes; saved
+ * and scratch 256-byte aligned. */
+int64_t alodlm_layer_saved(int64_t rows, int64_t hidden, int64_t nq, int64_t nkv, int64_t dh,
+                           int64_t inter, int dtype);
+int64_t alodlm_layer_fwd_scratch(int64_t rows, int64_t hidden, int64_t nq, int64_t nkv, int64_t dh,
+                                 int64_t inter, int dtype);
+int alodlm_layer_fwd(const void* x, const void* wqkv, const void* wo, const void* wgu,
+                     const void* wd, const void* ln1, const void* ln2, const void* qn,
+                     const void* kn, const void* cos_tab, const void* sin_tab,
+                     const int64_t* positions, const float* inv_freq, const int64_t* bounds,
+                     const int32_t* row_segment, const int32_t* tiles, int64_t n_tiles,
+                     int64_t block_size, void* k, void* v, void* saved, void* scratch, void* y,
+                     int64_t rows, int64_t hidden, int64_t nq, int64_t nkv,
+                     int64_t dh, int64_t inter, float eps, int dtype, void* stream);
+int64_t alodlm_layer_bwd_scratch(int64_t rows, int64_t hidden, int64_t nq, int64_t nkv, int64_t dh,
+                                 int64_t inter, int64_t n_tiles, int64_t ds_blocks, int dtype);
+int alodlm_layer_bwd(const void* dy, const void* x, const void* k, const void* saved,
+                     const void* wqkv, const void* wo, const void* wgu, const void* wd,
+                     const void* ln1, const void* ln2, const void* qn, const void* kn,
+                     const void* cos_tab, const void* sin_tab, const int64_t* positions,
+                     const float* inv_freq, const int64_t* bounds, const int32_t* row_segment,
+                     const int32_t* tiles, int64_t n_tiles, const int64_t* ds_base,
+                     int64_t ds_blocks, int64_t block_size, void* dwqkv, void* dwo, void* dwgu,
+                     void* dwd, float* dln1, float* dln2, float* dqn, float* dkn, void* scratch,
+                     void* dx, int64_t rows, int64_t hidden, int64_t nq, int64_t nkv, int64_t dh,
+                     int64_t inter, float eps, int dtype, void* stream);
+
 /* The weight gradient of a layer applied once per recurrent pass
  * (alodlm/model.py:152, the loop over depths, whose autograd sums the passes'
  * nn.Linear weight gradients) as one product:
