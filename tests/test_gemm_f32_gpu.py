@@ -1,6 +1,7 @@
 """The float32 matrix-core products through the C ABI against float64: every
-operand layout and epilogue at the edges of the 128x128 tiles and the 16-deep
-k stages, split and unsplit K, row strides wider than the rows.
+operand layout and epilogue at the edges of the 64x64 and 128x128 tiles (2044
+x 1924: one round of the large ones) and their 32- and 16-deep k stages, split
+and unsplit K, row strides wider than the rows.
 
 Bound: a float32 sum of K products of unit normals errs by at most K eps times
 the sum's absolute terms; in practice the partial sums grow like sqrt(k), which
@@ -17,7 +18,8 @@ DEV = "cuda"
 
 
 @pytest.mark.parametrize("M,N,K", [(72, 4, 4), (68, 132, 20), (128, 128, 16), (132, 260, 36),
-                                   (256, 128, 1000), (700, 384, 2048), (2048, 516, 700)])
+                                   (256, 128, 1000), (700, 384, 2048), (2048, 516, 700),
+                                   (2044, 1924, 52)])
 @pytest.mark.parametrize("ak,bk", [(1, 1), (1, 0), (0, 1), (0, 0)])
 @pytest.mark.parametrize("epi", [0, 1, 2, 3])
 def test_float32_products(M, N, K, ak, bk, epi):
