@@ -2,16 +2,19 @@
 //
 //   C[m, n] = alpha * sum_k A(m, k) * B(n, k)
 //
-// bf16 path: 128x128x64 tiles, 4 wavefronts in a 2x2 grid, each computing a
-// 64x64 block with v_mfma_f32_32x32x16_bf16.  Operands are staged through LDS
+// bf16: few rows go to gemm_skinny.hip, the rest to the 256x256 tiles of
+// gemm_dl.hip or the 128-column tiles of gemm_mid.hip (bf16_plan, below).  What
+// none of them takes (unaligned operands, small float outputs) runs in
+// gemm_big.hip or on the tiles of this file: 128x128x64, 4 wavefronts in a 2x2
+// grid, each computing a 64x64 block with v_mfma_f32_32x32x16_bf16.  Operands are staged through LDS
 // in k-contiguous rows (padded by 8 elements); an operand stored m/n-contiguous
 // ([K, M] in memory, as in the backward's dW and dX products) is transposed
 // while it is staged: each thread loads an 8(k) x 4(m) block with 8-byte
 // loads and writes four 16-byte k-rows.  Global loads for tile k+1 are issued
 // before the MFMAs of tile k (register prefetch, double-buffered LDS).
 //
-// float: gemm_f32.hip; few rows: gemm_skinny.hip; unaligned shapes: a plain
-// LDS-tiled FMA kernel.
+// float: gemm_skinny.hip (few rows) and gemm_f32.hip; unaligned operands: a
+// plain LDS-tiled FMA kernel.
 #include <type_traits>
 
 #include "common.h"
@@ -505,11 +508,14 @@ extern "C" int alodlm_gemm(const void* A, int64_t lda, int a_kmajor, const void*
                      gemm_dl_eligible(lda, a_kmajor, ldb, b_kmajor, M, N, K);
   const bool mid_ok = dtype == ALODLM_BF16 &&
                       gemm_mid_eligible(A, lda, a_kmajor, B, ldb, b_kmajor, M, N, K);
-  // few rows: up to one 16-row block stream the weight without LDS; above that
-  // the bf16 tiles of 32 or 64 rows, which share A between their waves, are as
-  // fast or faster (27 rows, 4096 x 12288: 27 us against 38; 4096 x 4096: 12.2
-  // against 13.5; 16 rows, 4096 x 2048: 9.6 against 6.3)
-  if ((dtype == ALODLM_F32 || (dtype == ALODLM_BF16 && (M <= 16 || !mid_ok))) &&
+  // few rows: float, one block of 16 bf16 rows, and up to 48 over at most one
+  // 16-row workgroup per CU (48 rows up to K = 8192, where re-reading A weighs
+  // less) stream the weight; the bf16 tiles of 32 or 64 rows, which share A
+  // between their waves, take the rest (27 rows, 4096 x 4096: 9.1 us against
+  // 12.2; 48 rows, 2048 x 6144: 11.8 against 14.7, 4096 x 12288: 33.6 against 29;
+  // 27 rows, 24576 x 4096: 51 against 46)
+  const bool narrow = N <= 16 * 256 && (M <= 32 || (M <= 48 && K <= 8192));
+  if ((dtype == ALODLM_F32 || (dtype == ALODLM_BF16 && (M <= 16 || narrow || !mid_ok))) &&
       gemm_skinny_eligible(A, lda, a_kmajor, B, ldb, b_kmajor, M, N, K, epilogue, dtype)) {
     gemm_skinny_launch(A, lda, B, ldb, C, ldc, R, ldr, M, N, K, alpha, epilogue, dtype, st);
     ALODLM_CHECK_LAUNCH("gemm_skinny");

@@ -22,7 +22,7 @@ DEV = "cuda"
 @pytest.mark.parametrize("M,N,K", [
     (1, 16, 8), (5, 33, 40), (16, 4096, 2048), (16, 12304, 264), (17, 4112, 520),
     (32, 130, 2056), (33, 6144, 1032), (48, 2048, 6144), (49, 50, 4104), (64, 96, 1024),
-    (65, 96, 1024)])
+    (65, 96, 1024), (9, 4130, 776), (20, 1000, 72), (48, 4096, 8200)])
 @pytest.mark.parametrize("epi", [0, 1])
 def test_few_rows(M, N, K, dtype, epi):
     log(f"gemm few rows M={M} N={N} K={K} {dtype} epi={epi}")
