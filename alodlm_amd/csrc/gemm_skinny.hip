@@ -15,7 +15,7 @@
 // load touch 16 lines, which a CU's address path serves at about 30 KB/us; 8
 // consecutive lanes per line reach 58.  16 rows, bf16, direct to registers and
 // now: 4096 x 2048 6.3 and 5.9 us, 2048 x 2048 5.8 and 4.8, 2048 x 6144 12.8 and
-// 7.4, 12288 x 2048 14.4 and 12.7; float 2048 x 6144 24.3 and 17.5, 48 rows of
+// 7.6, 12288 x 2048 14.3 and 12.1; float 2048 x 6144 24.3 and 17.5, 48 rows of
 // 4096 x 12288 101 and 65.
 //
 // Fragment: lane l holds 16 bytes of row l % 16 at 16-byte chunk l / 16.  For

@@ -2,7 +2,7 @@
 // alodlm/inference.py:83-88, and a differentiable call's forward and
 // backward): the launches of the steps below are enqueued without returning
 // to the caller between them, over one scratch allocation whose regions the
-// steps share.  16 window rows keep the chip busy for 66 us per layer, and the
+// steps share.  16 window rows keep the chip busy for 57 us per layer, and the
 // separate calls with their output allocations took 95 us of host time, 36 us
 // now.  Forward and backward of a 1.7B layer over 300 rows: 530 us a call and
 // 440 now, with about 400 us of kernels; 2474 rows 1213 and 1199.
