@@ -11,7 +11,7 @@ from pathlib import Path
 import torch
 
 LIBRARY = Path(__file__).resolve().parent / "libalodlm_hip.so"
-ABI_VERSION = 7
+ABI_VERSION = 8
 
 P = ctypes.c_void_p
 I64 = ctypes.c_int64
@@ -39,9 +39,10 @@ SIGNATURES = {
                            + [F32, I32, P],
     "alodlm_layer_saved": [I64] * 6 + [I32],
     "alodlm_layer_fwd_scratch": [I64] * 6 + [I32],
-    "alodlm_layer_fwd": [P] * 16 + [I64, I64] + [P] * 5 + [I64] * 6 + [F32, I32, P],
+    "alodlm_layer_fwd": [P] * 16 + [I64, I64] + [P] * 5 + [I64] * 6 + [F32, I32, I32, P],
     "alodlm_layer_bwd_scratch": [I64] * 8 + [I32],
-    "alodlm_layer_bwd": [P] * 19 + [I64, P, I64, I64] + [P] * 10 + [I64] * 6 + [F32, I32, P],
+    "alodlm_layer_bwd": [P] * 19 + [I64, P, I64, I64] + [P] * 10 + [I64] * 6
+                        + [F32, I32, I32, P],
     "alodlm_rmsnorm_bwd_workspace": [I64, I64],
     "alodlm_embed_plan_size": [I64],
     "alodlm_embed_scatter_workspace": [I64, I64],
@@ -60,6 +61,8 @@ SIGNATURES = {
     "alodlm_rotary_bwd": [P, P, P, P, I64, I64, I64, I32, P],
     "alodlm_gemm_workspace": [I64, I64, I64, I32, I32],
     "alodlm_gemm": [P, I64, I32, P, I64, I32, P, I64, P, I64, I64, I64, I64, F32, I32, I32, P, P],
+    "alodlm_gemm_chain": [P, I64, I32, P, I64, I32, P, I64, P, I64, I64, I64, I64, F32, I32, I32, P,
+                          P],
     "alodlm_gemm_segk": [P, P, I32, I64, I64, I64, P, I64, I64, I64, F32, I32, P, P],
     "alodlm_attention_fwd": [P, P, P, I64, P, P, P, I64, P, P, I64, I64, I64, I64, I64, I32, P],
     "alodlm_attention_ds_blocks": [P, I64, I64, P],

@@ -14,6 +14,7 @@
 // dK/dV pass; the wavefront spreads head_dim over its lanes.
 #include <initializer_list>
 
+#include "attention.h"
 #include "attention_common.h"
 
 #define ATT_MAX_PER_LANE 4  // head_dim <= 256
@@ -253,11 +254,10 @@ static bool use_mfma(int dtype, int64_t dh, const int32_t* tiles, int64_t ldv,
 // share the keys (attention_few.hip).
 constexpr int64_t FEW_WORKGROUPS = 256;
 
-extern "C" int alodlm_attention_fwd(const void* q, const void* k, const void* v, int64_t ldv,
-                                    const int64_t* bounds, const int32_t* row_segment,
-                                    const int32_t* tiles, int64_t n_tiles, void* o, float* lse,
-                                    int64_t rows, int64_t nq, int64_t nkv, int64_t dh,
-                                    int64_t block_size, int dtype, void* stream) {
+int attention_fwd(const void* q, const void* k, const void* v, int64_t ldv, const int64_t* bounds,
+                  const int32_t* row_segment, const int32_t* tiles, int64_t n_tiles, void* o,
+                  float* lse, int64_t rows, int64_t nq, int64_t nkv, int64_t dh,
+                  int64_t block_size, int dtype, bool chain, void* stream) {
   int rc = check_attn(rows, nq, nkv, dh, block_size);
   if (rc) return rc;
   if (rows == 0) return ALODLM_OK;
@@ -265,7 +265,7 @@ extern "C" int alodlm_attention_fwd(const void* q, const void* k, const void* v,
   if (use_mfma(dtype, dh, tiles, ldv, {q, k, v, o})) {
     if (n_tiles == 0) return ALODLM_OK;
     ALODLM_CHECK_ARG(n_tiles <= 65535, "attention: too many 128-row tiles (%lld)", (long long)n_tiles);
-    if (dh == 128 && n_tiles * nq < FEW_WORKGROUPS && 4 * n_tiles <= 65535) {
+    if (dh == 128 && !chain && n_tiles * nq < FEW_WORKGROUPS && 4 * n_tiles <= 65535) {
       fa128_few_launch((const bf16_t*)q, (const bf16_t*)k, (const bf16_t*)v, ldv, bounds, tiles,
                        n_tiles, (bf16_t*)o, lse, rows, (int)nq, (int)nkv, (int)block_size, scale,
                        as_stream(stream));
@@ -294,6 +294,15 @@ extern "C" int alodlm_attention_fwd(const void* q, const void* k, const void* v,
   });
   ALODLM_CHECK_LAUNCH("attention_fwd");
   return ALODLM_OK;
+}
+
+extern "C" int alodlm_attention_fwd(const void* q, const void* k, const void* v, int64_t ldv,
+                                    const int64_t* bounds, const int32_t* row_segment,
+                                    const int32_t* tiles, int64_t n_tiles, void* o, float* lse,
+                                    int64_t rows, int64_t nq, int64_t nkv, int64_t dh,
+                                    int64_t block_size, int dtype, void* stream) {
+  return attention_fwd(q, k, v, ldv, bounds, row_segment, tiles, n_tiles, o, lse, rows, nq, nkv, dh,
+                       block_size, dtype, false, stream);
 }
 
 int64_t fa128_bwd_workspace(int64_t N, int nq, int nkv, int64_t n_tiles, int64_t ds_blocks);

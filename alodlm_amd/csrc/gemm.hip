@@ -494,10 +494,15 @@ static void launch_mfma(const bf16_t* A, int64_t lda, const bf16_t* B, int64_t l
   if (part) splitk_reduce(part, nsplit, M, N, C, ldc, nullptr, 0, epi, ALODLM_BF16, st);
 }
 
-extern "C" int alodlm_gemm(const void* A, int64_t lda, int a_kmajor, const void* B, int64_t ldb,
-                           int b_kmajor, void* C, int64_t ldc, const void* R, int64_t ldr,
-                           int64_t M, int64_t N, int64_t K, float alpha, int epilogue, int dtype,
-                           float* workspace, void* stream) {
+// `chain` (bf16): every output is one chain of MFMA steps in k order, which all
+// the tiles give the same bits for (their instructions differ in shape, not in
+// the order they add k in), so neither the few-row kernel, whose waves share K,
+// nor a split of K is taken; only the long-K products of the 256x256 tiles
+// (gemm_dl_store_splits) keep theirs.
+static int gemm_dispatch(const void* A, int64_t lda, int a_kmajor, const void* B, int64_t ldb,
+                         int b_kmajor, void* C, int64_t ldc, const void* R, int64_t ldr, int64_t M,
+                         int64_t N, int64_t K, float alpha, int epilogue, int dtype, bool chain,
+                         float* workspace, void* stream) {
   ALODLM_CHECK_ARG(M >= 0 && N >= 0 && K >= 0, "gemm: negative shape");
   ALODLM_CHECK_ARG(epilogue >= 0 && epilogue <= 3, "gemm: bad epilogue");
   ALODLM_CHECK_ARG(epilogue != ALODLM_EPI_RESIDUAL || R != nullptr, "gemm: residual needs R");
@@ -515,13 +520,16 @@ extern "C" int alodlm_gemm(const void* A, int64_t lda, int a_kmajor, const void*
   // 12.2; 48 rows, 2048 x 6144: 11.8 against 14.7, 4096 x 12288: 33.6 against 29;
   // 27 rows, 24576 x 4096: 51 against 46)
   const bool narrow = N <= 16 * 256 && (M <= 32 || (M <= 48 && K <= 8192));
-  if ((dtype == ALODLM_F32 || (dtype == ALODLM_BF16 && (M <= 16 || narrow || !mid_ok))) &&
+  if ((dtype == ALODLM_F32 || (dtype == ALODLM_BF16 && !chain && (M <= 16 || narrow || !mid_ok))) &&
       gemm_skinny_eligible(A, lda, a_kmajor, B, ldb, b_kmajor, M, N, K, epilogue, dtype)) {
     gemm_skinny_launch(A, lda, B, ldb, C, ldc, R, ldr, M, N, K, alpha, epilogue, dtype, st);
     ALODLM_CHECK_LAUNCH("gemm_skinny");
     return ALODLM_OK;
   }
-  const Bf16Plan plan = bf16_plan(M, N, K, epilogue, a_kmajor, dl_ok, mid_ok, workspace != nullptr);
+  const bool long_k = chain && dl_ok && epilogue == ALODLM_EPI_STORE && K >= 16384;
+  const Bf16Plan plan =
+      long_k ? Bf16Plan{false, workspace ? gemm_dl_store_splits(M, N, K) : 1, 0.0}
+             : bf16_plan(M, N, K, epilogue, a_kmajor, dl_ok, mid_ok, workspace != nullptr && !chain);
   if (mid_ok && plan.mid) {
     const int64_t nsplit = gemm_mid_launch((const bf16_t*)A, lda, a_kmajor, (const bf16_t*)B, ldb,
                                            b_kmajor, C, ldc, (const bf16_t*)R, ldr, M, N, K, alpha,
@@ -626,6 +634,24 @@ extern "C" int alodlm_gemm(const void* A, int64_t lda, int a_kmajor, const void*
   });
   ALODLM_CHECK_LAUNCH("gemm_simple");
   return ALODLM_OK;
+}
+
+extern "C" int alodlm_gemm(const void* A, int64_t lda, int a_kmajor, const void* B, int64_t ldb,
+                           int b_kmajor, void* C, int64_t ldc, const void* R, int64_t ldr,
+                           int64_t M, int64_t N, int64_t K, float alpha, int epilogue, int dtype,
+                           float* workspace, void* stream) {
+  return gemm_dispatch(A, lda, a_kmajor, B, ldb, b_kmajor, C, ldc, R, ldr, M, N, K, alpha, epilogue,
+                       dtype, false, workspace, stream);
+}
+
+extern "C" int alodlm_gemm_chain(const void* A, int64_t lda, int a_kmajor, const void* B,
+                                 int64_t ldb, int b_kmajor, void* C, int64_t ldc, const void* R,
+                                 int64_t ldr, int64_t M, int64_t N, int64_t K, float alpha,
+                                 int epilogue, int dtype, float* workspace, void* stream) {
+  ALODLM_CHECK_ARG(epilogue == ALODLM_EPI_STORE || epilogue == ALODLM_EPI_RESIDUAL,
+                   "gemm_chain: an output of the storage type");
+  return gemm_dispatch(A, lda, a_kmajor, B, ldb, b_kmajor, C, ldc, R, ldr, M, N, K, alpha, epilogue,
+                       dtype, true, workspace, stream);
 }
 
 extern "C" int alodlm_gemm_segk(const void* const* a_segs, const void* const* b_segs, int nseg,

@@ -8,6 +8,7 @@
 // 440 now, with about 400 us of kernels; 2474 rows 1213 and 1199.
 #include <algorithm>
 
+#include "attention.h"
 #include "common.h"
 
 namespace {
@@ -26,6 +27,7 @@ struct Layer {
   int dtype;
   float eps;
   void* stream;
+  bool chain = false;  // products and attention as alodlm_gemm_chain sums them
   int64_t es() const { return dtype == ALODLM_BF16 ? 2 : 4; }
   int64_t QD() const { return nq * dh; }
   int64_t KD() const { return nkv * dh; }
@@ -39,14 +41,14 @@ struct Layer {
   int product(const void* A, const void* w, const void* w_t, void* C, int64_t N, int64_t K,
               const void* R, float* ws) const {
     const bool copy = w_t != nullptr && rows > SKINNY_ROWS;
-    return alodlm_gemm(A, K, 1, copy ? w_t : w, copy ? N : K, copy ? 0 : 1, C, N, R, R ? N : 0,
-                       rows, N, K, 1.f, R ? ALODLM_EPI_RESIDUAL : ALODLM_EPI_STORE, dtype, ws,
-                       stream);
+    return (chain ? alodlm_gemm_chain : alodlm_gemm)(
+        A, K, 1, copy ? w_t : w, copy ? N : K, copy ? 0 : 1, C, N, R, R ? N : 0, rows, N, K, 1.f,
+        R ? ALODLM_EPI_RESIDUAL : ALODLM_EPI_STORE, dtype, ws, stream);
   }
   // dA = dC w for the product above
   int input_grad(const void* dC, const void* w, void* dA, int64_t N, int64_t K, float* ws) const {
-    return alodlm_gemm(dC, N, 1, w, K, 0, dA, K, nullptr, 0, rows, K, N, 1.f, ALODLM_EPI_STORE,
-                       dtype, ws, stream);
+    return (chain ? alodlm_gemm_chain : alodlm_gemm)(dC, N, 1, w, K, 0, dA, K, nullptr, 0, rows, K,
+                                                     N, 1.f, ALODLM_EPI_STORE, dtype, ws, stream);
   }
   // dw = dC^T A, in the storage dtype
   int weight_grad(const void* dC, const void* A, void* dw, int64_t N, int64_t K, float* ws) const {
@@ -229,8 +231,8 @@ extern "C" int alodlm_layer_fwd(const void* x, const void* wqkv, const void* wo,
                                 const int32_t* tiles, int64_t n_tiles, int64_t block_size, void* k,
                                 void* v, void* saved, void* scratch, void* y, int64_t rows,
                                 int64_t hidden, int64_t nq, int64_t nkv, int64_t dh, int64_t inter,
-                                float eps, int dtype, void* stream) {
-  const Layer l{rows, hidden, nq, nkv, dh, inter, dtype, eps, stream};
+                                float eps, int chain, int dtype, void* stream) {
+  const Layer l{rows, hidden, nq, nkv, dh, inter, dtype, eps, stream, chain != 0};
   ALODLM_CHECK_ARG(l.ok(), "layer_fwd: bad shape or dtype");
   ALODLM_CHECK_ARG(rows == 0 || (cos_tab ? sin_tab && v : positions && inv_freq && !v),
                    "layer_fwd: needs rotary tables with v, or positions without");
@@ -251,8 +253,8 @@ extern "C" int alodlm_layer_fwd(const void* x, const void* wqkv, const void* wo,
     v = static_cast<char*>(m[s.qkv]) + (l.QD() + l.KD()) * l.es();
     ldv = l.W();
   }
-  RUN(alodlm_attention_fwd(m[s.q], k, v, ldv, bounds, row_segment, tiles, n_tiles, m[s.o],
-                           m.floats(s.lse), rows, nq, nkv, dh, block_size, dtype, stream));
+  RUN(attention_fwd(m[s.q], k, v, ldv, bounds, row_segment, tiles, n_tiles, m[s.o],
+                    m.floats(s.lse), rows, nq, nkv, dh, block_size, dtype, l.chain, stream));
   RUN(l.product(m[s.o], wo, nullptr, m[s.x1], l.H, l.QD(), x, ws));
   RUN(l.norm(m[s.x1], ln2, h, m.floats(s.rstd2)));
   RUN(l.product(h, wgu, nullptr, m[s.gu], 2 * l.I, l.H, nullptr, ws));
@@ -275,9 +277,9 @@ extern "C" int alodlm_layer_bwd(
     const int32_t* row_segment, const int32_t* tiles, int64_t n_tiles, const int64_t* ds_base,
     int64_t ds_blocks, int64_t block_size, void* dwqkv, void* dwo, void* dwgu, void* dwd,
     float* dln1, float* dln2, float* dqn, float* dkn, void* scratch, void* dx, int64_t rows,
-    int64_t hidden, int64_t nq, int64_t nkv, int64_t dh, int64_t inter, float eps, int dtype,
-    void* stream) {
-  const Layer l{rows, hidden, nq, nkv, dh, inter, dtype, eps, stream};
+    int64_t hidden, int64_t nq, int64_t nkv, int64_t dh, int64_t inter, float eps, int chain,
+    int dtype, void* stream) {
+  const Layer l{rows, hidden, nq, nkv, dh, inter, dtype, eps, stream, chain != 0};
   ALODLM_CHECK_ARG(l.ok(), "layer_bwd: bad shape or dtype");
   ALODLM_CHECK_ARG(rows == 0 || (cos_tab ? sin_tab != nullptr : positions && inv_freq),
                    "layer_bwd: needs rotary tables or positions");

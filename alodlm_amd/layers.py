@@ -325,12 +325,12 @@ class Kernels:
              ptr(dtable), ptr(ws), N, H, dtable.shape[0], self.code, self._stream())
 
     def _gemm(self, A, lda, a_k, B, ldb, b_k, C, ldc, M, N, K, alpha=1.0, epi=EPI_STORE, R=None,
-              ldr=0):
+              ldr=0, chain=False):
         ws = None
         need = query("alodlm_gemm_workspace", M, N, K, epi, self.code)
         if need:
             ws = self._workspace(need)
-        call("alodlm_gemm", ptr(A), lda, a_k, ptr(B), ldb, b_k, ptr(C), ldc, ptr(R), ldr, M, N, K,
+        call("alodlm_gemm_chain" if chain else "alodlm_gemm", ptr(A), lda, a_k, ptr(B), ldb, b_k, ptr(C), ldc, ptr(R), ldr, M, N, K,
              alpha, epi, self.code, ptr(ws), self._stream())
 
     def _product(self, x, ldx, w, w_t, y, M, N, K, epi=EPI_STORE, R=None, ldr=0):
@@ -532,10 +532,11 @@ class Kernels:
     def _bytes(self, size, *args):
         return torch.empty(query(size, *args), dtype=torch.uint8, device=self.device)
 
-    def layer_call_fwd(self, w, x, rope, mask):
+    def layer_call_fwd(self, w, x, rope, mask, chain=False):
         """One differentiable layer call over x [N, H] as one host call
         (``layer_fwd``'s steps): returns y, the rotated keys, the values (None
-        without rotary tables) and the bytes ``layer_call_bwd`` reads."""
+        without rotary tables) and the bytes ``layer_call_bwd`` reads.  With
+        ``chain`` a row's sums run in one order whatever the other rows."""
         d, N = self.dims, x.shape[0]
         dims = self._layer_dims(N)
         saved = self._bytes("alodlm_layer_saved", *dims, self.code)
@@ -547,10 +548,10 @@ class Kernels:
              ptr(w.ln2), ptr(w.qn), ptr(w.kn), ptr(rope.cos), ptr(rope.sin), ptr(rope.positions),
              ptr(rope.inv_freq), ptr(mask.boundaries), ptr(mask.row_segment), ptr(mask.tiles),
              0 if mask.tiles is None else mask.tiles.shape[0], mask.block_size, ptr(k), ptr(v),
-             ptr(saved), ptr(scratch), ptr(y), *dims, d.eps, self.code, self._stream())
+             ptr(saved), ptr(scratch), ptr(y), *dims, d.eps, chain, self.code, self._stream())
         return y, k, v, saved
 
-    def layer_call_bwd(self, dy, x, k, saved, w, gw, rope, mask):
+    def layer_call_bwd(self, dy, x, k, saved, w, gw, rope, mask, chain=False):
         """Backward of ``layer_call_fwd``: returns dx, writes the matrices'
         gradients (``gw.stored``) and adds the norm weights' to ``gw``."""
         d, dims = self.dims, self._layer_dims(x.shape[0])
@@ -564,7 +565,7 @@ class Kernels:
              ptr(mask.row_segment), ptr(mask.tiles), n_tiles,
              ptr(getattr(mask, "ds_base", None)), ds_blocks, mask.block_size, ptr(gw.wqkv),
              ptr(gw.wo), ptr(gw.wgu), ptr(gw.wd), ptr(gw.ln1), ptr(gw.ln2), ptr(gw.qn), ptr(gw.kn),
-             ptr(scratch), ptr(dx), *dims, d.eps, self.code, self._stream())
+             ptr(scratch), ptr(dx), *dims, d.eps, chain, self.code, self._stream())
         return dx
 
 
@@ -620,10 +621,11 @@ class _LayerFunction(torch.autograd.Function):
     """training_layer / layer_forward as one autograd node over the kernels."""
 
     @staticmethod
-    def forward(ctx, kernels, mask, rope, hidden, *params):
+    def forward(ctx, kernels, mask, rope, chain, hidden, *params):
         w = LayerWeights.from_tensors(*params)
         x = hidden.contiguous()
-        y, k, v, saved = kernels.layer_call_fwd(w, x, rope, mask)
+        y, k, v, saved = kernels.layer_call_fwd(w, x, rope, mask, chain)
+        ctx.chain = chain
         ctx.kernels, ctx.mask, ctx.rope, ctx.saved, ctx.w = kernels, mask, rope, (x, k, saved), w
         ctx.shapes = [(p.shape, p.dtype) for p in params]
         if v is None:  # only a table-driven call hands its keys and values out
@@ -643,7 +645,8 @@ class _LayerFunction(torch.autograd.Function):
                         mats[3].view(H, I), *norms.split([H, H, d.head_dim, d.head_dim]),
                         stored=True)
         x, k, saved = ctx.saved
-        dx = kernels.layer_call_bwd(dy.contiguous(), x, k, saved, w, gw, ctx.rope, ctx.mask)
+        dx = kernels.layer_call_bwd(dy.contiguous(), x, k, saved, w, gw, ctx.rope, ctx.mask,
+                                    ctx.chain)
         ctx.saved = None
         if len({dtype for _, dtype in ctx.shapes[7:]}) == 1:  # one cast for the four
             norms = norms.to(ctx.shapes[7][1])
@@ -651,7 +654,7 @@ class _LayerFunction(torch.autograd.Function):
         parts = [gw.wqkv[:qd], gw.wqkv[qd:qd + kd], gw.wqkv[qd + kd:], gw.wo, gw.wgu[:I],
                  gw.wgu[I:], gw.wd, *norms.split([H, H, d.head_dim, d.head_dim])]
         grads = [g.view(shape).to(dtype) for g, (shape, dtype) in zip(parts, ctx.shapes)]
-        return (None, None, None, dx, *grads)
+        return (None, None, None, None, dx, *grads)
 
 
 class _Rotary(torch.autograd.Function):

@@ -89,7 +89,9 @@ class _AutoregressiveLoss(torch.autograd.Function):
         src = logits.detach().contiguous()
         coef = torch.full((R,), 1.0 / R, dtype=torch.float32, device=dev)
         ce = torch.empty(R, dtype=torch.float32, device=dev)
-        # ce[r] = logsumexp - logit[target]; buf <- (softmax - onehot) / R
+        # ce[r] = logsumexp - logit[target] in float32 for bf16 logits too: rounding
+        # each term to bf16 first adds up to 2^-9 of it, which the mean of a few
+        # hundred terms leaves at about 5e-5 of the loss; buf <- (softmax - onehot) / R
         call("alodlm_cross_entropy_rows", ptr(src), ptr(sel), ptr(buf), ptr(target), ptr(coef),
              ptr(n_rows), R, V, ptr(ce), None, _lib.dtype_code(logits.dtype),
              _lib.stream_handle(dev))

@@ -99,7 +99,7 @@ def layer_forward(layer, hidden, cos, sin, mask, prefix=None):
     _check_device(hidden, "layer_forward")
     kind = _kernel_mask(mask, L, hidden.device)
     if prefix is None and not (isinstance(kind, tuple) and kind[0] == "window"):
-        y, k, v = _LayerFunction.apply(kernels, kind, rope, hidden,
+        y, k, v = _LayerFunction.apply(kernels, kind, rope, False, hidden,
                                        *LayerWeights.module_tensors(layer))
         return y, (k, v)
     P = kind[1] if isinstance(kind, tuple) else None

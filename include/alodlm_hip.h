@@ -27,7 +27,7 @@
 extern "C" {
 #endif
 
-#define ALODLM_ABI_VERSION 7
+#define ALODLM_ABI_VERSION 8
 
 enum { ALODLM_OK = 0, ALODLM_EINVAL = 1, ALODLM_EHIP = 2, ALODLM_EUNSUPPORTED = 3 };
 enum { ALODLM_F32 = 0, ALODLM_BF16 = 1 };
@@ -215,6 +215,14 @@ int alodlm_gemm(const void* A, int64_t lda, int a_kmajor, const void* B, int64_t
                 int b_kmajor, void* C, int64_t ldc, const void* R, int64_t ldr, int64_t M,
                 int64_t N, int64_t K, float alpha, int epilogue, int dtype, float* workspace,
                 void* stream);
+/* alodlm_gemm (STORE or RESIDUAL) with every bf16 output summed as one chain in
+ * k order, so that a row's bits do not depend on how many rows the product has:
+ * K is neither split nor shared between waves, but for STORE products of M, N
+ * >= 256 and K >= 16384 as above.  float32: the same as alodlm_gemm. */
+int alodlm_gemm_chain(const void* A, int64_t lda, int a_kmajor, const void* B, int64_t ldb,
+                      int b_kmajor, void* C, int64_t ldc, const void* R, int64_t ldr, int64_t M,
+                      int64_t N, int64_t K, float alpha, int epilogue, int dtype,
+                      float* workspace, void* stream);
 /* C = rmsnorm(x) . W^T for at most 16 bf16 rows (alodlm/model.py:56-58,75 in a
  * decoding window): x [M, K] of row stride ldx, W [N, K]; with `swiglu` W's rows
  * are the gate then the up projection and C [M, N/2] = silu(gate) * up.  Each
@@ -251,7 +259,9 @@ int alodlm_window_layer(
  * (alodlm_layer_saved(...) bytes).  Backward: dx, the matrices' gradients in
  * the storage dtype (written), the norm weights' in float32 (added).
  * scratch: alodlm_layer_fwd_scratch(...) and _bwd_scratch(...) bytes; saved
- * and scratch 256-byte aligned. */
+ * and scratch 256-byte aligned.  With `chain` (bf16) the layer's products are
+ * alodlm_gemm_chain's and each row's attention runs over its keys in one order,
+ * so y does not depend on the other rows of the call. */
 int64_t alodlm_layer_saved(int64_t rows, int64_t hidden, int64_t nq, int64_t nkv, int64_t dh,
                            int64_t inter, int dtype);
 int64_t alodlm_layer_fwd_scratch(int64_t rows, int64_t hidden, int64_t nq, int64_t nkv, int64_t dh,
@@ -262,8 +272,8 @@ int alodlm_layer_fwd(const void* x, const void* wqkv, const void* wo, const void
                      const int64_t* positions, const float* inv_freq, const int64_t* bounds,
                      const int32_t* row_segment, const int32_t* tiles, int64_t n_tiles,
                      int64_t block_size, void* k, void* v, void* saved, void* scratch, void* y,
-                     int64_t rows, int64_t hidden, int64_t nq, int64_t nkv,
-                     int64_t dh, int64_t inter, float eps, int dtype, void* stream);
+                     int64_t rows, int64_t hidden, int64_t nq, int64_t nkv, int64_t dh,
+                     int64_t inter, float eps, int chain, int dtype, void* stream);
 int64_t alodlm_layer_bwd_scratch(int64_t rows, int64_t hidden, int64_t nq, int64_t nkv, int64_t dh,
                                  int64_t inter, int64_t n_tiles, int64_t ds_blocks, int dtype);
 int alodlm_layer_bwd(const void* dy, const void* x, const void* k, const void* saved,
@@ -275,7 +285,7 @@ int alodlm_layer_bwd(const void* dy, const void* x, const void* k, const void* s
                      int64_t ds_blocks, int64_t block_size, void* dwqkv, void* dwo, void* dwgu,
                      void* dwd, float* dln1, float* dln2, float* dqn, float* dkn, void* scratch,
                      void* dx, int64_t rows, int64_t hidden, int64_t nq, int64_t nkv, int64_t dh,
-                     int64_t inter, float eps, int dtype, void* stream);
+                     int64_t inter, float eps, int chain, int dtype, void* stream);
 
 /* The weight gradient of a layer applied once per recurrent pass
  * (alodlm/model.py:152, the loop over depths, whose autograd sums the passes'
