@@ -708,6 +708,14 @@ class WindowSlot:
             raise ValueError("the window slot belongs to another layer")
         if self.k.shape[0] < P + L or self.v.shape[0] < P + L or L != self.mask.window:
             raise ValueError("the window does not fit the slot's cache rows")
+        # the kernels take whole contiguous rows of the storage dtype
+        if hidden.dtype != self.kernels.dtype:
+            raise ValueError(f"hidden must be {self.kernels.dtype}, got {hidden.dtype}")
+        for t in (self.k, self.v):
+            if (t.dtype != hidden.dtype or t.device != hidden.device or not t.is_contiguous()
+                    or t.numel() != t.shape[0] * d.kv_heads * d.head_dim):
+                raise ValueError(f"the slot's buffers must be contiguous [rows, {d.kv_heads}, "
+                                 f"{d.head_dim}] {hidden.dtype} tensors on {hidden.device}")
         rope = Rope(cos=table(cos, L, d.head_dim, hidden), sin=table(sin, L, d.head_dim, hidden))
         y = self.kernels.layer_window(self.weights, hidden.contiguous(), rope, self.mask,
                                       self.k, self.v)

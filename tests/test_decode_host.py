@@ -132,3 +132,43 @@ def test_stop_tokens_and_penalty():
     assert stop_token_ids(Tok(None, {})) == []
     assert DecodeConfig(tau=0.4).penalty == pytest.approx(0.02)
     assert DecodeConfig(tau=0.4, position_penalty=0.0).penalty == 0.0
+
+
+def test_window_slot_rejects_buffers_the_kernels_cannot_address():
+    """A slot's buffers are read and written as contiguous rows of
+    kv_heads * head_dim values of the model's dtype: a strided cache, another
+    dtype or another row width raises ValueError before any kernel runs; views
+    of whole rows pass."""
+    from types import SimpleNamespace
+    from alodlm_amd.layers import WindowSlot
+    P, L, nkv, dh, H = 5, 3, 2, 4, 16
+    ran = []
+
+    def layer_window(w, x, rope, mask, k, v):
+        ran.append((k, v))
+        return x
+    kernels = SimpleNamespace(dims=SimpleNamespace(kv_heads=nkv, head_dim=dh), dtype=torch.float32,
+                              layer_window=layer_window)
+    q = torch.zeros(4, H)
+    layer = SimpleNamespace(self_attn=SimpleNamespace(q_proj=SimpleNamespace(weight=q)))
+    mask = SimpleNamespace(prefix=P, window=L)
+    hidden, table = torch.zeros(L, H), torch.zeros(L, dh)
+    buf = lambda: torch.zeros(10, nkv, dh)
+
+    def run(k, v, hidden=hidden):
+        return WindowSlot(kernels, SimpleNamespace(wqkv=q), k, v, mask).run(layer, hidden, table,
+                                                                          table)
+    by_layer = torch.zeros(10, 3, nkv, dh)  # [capacity, layers, ...] indexed by layer
+    for bad in (by_layer[:, 1], torch.zeros(20, nkv, dh)[::2], buf().to(torch.bfloat16),
+                torch.zeros(10, nkv, dh - 1), torch.zeros(10, nkv + 1, dh), buf().to("meta")):
+        with pytest.raises(ValueError, match="buffers must be contiguous"):
+            run(bad, buf())
+        with pytest.raises(ValueError, match="buffers must be contiguous"):
+            run(buf(), bad)
+    with pytest.raises(ValueError, match="hidden must be"):
+        run(buf(), buf(), hidden.to(torch.bfloat16))
+    assert not ran
+    k, v = torch.zeros(12, nkv, dh)[2:], torch.zeros(10, nkv * dh)
+    y, (k_rows, v_rows) = run(k, v)
+    assert len(ran) == 1 and ran[0][0] is k and ran[0][1] is v
+    assert k_rows.data_ptr() == k[P:].data_ptr() and k_rows.shape[0] == L
