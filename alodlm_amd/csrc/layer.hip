@@ -181,7 +181,8 @@ extern "C" int alodlm_window_layer(
   const Layer l{rows, hidden, nq, nkv, dh, inter, dtype, eps, stream};
   ALODLM_CHECK_ARG(l.ok(), "window_layer: bad shape or dtype");
   ALODLM_CHECK_ARG(rows == 0 || (cos_tab && sin_tab), "window_layer: needs rotary tables");
-  ALODLM_CHECK_ARG(prefix >= 0 && base >= 0 && base <= prefix, "window_layer: bad prefix");
+  // the query rows start at the window, so the mask's row 0 is key row `prefix`
+  ALODLM_CHECK_ARG(prefix >= 0 && base == prefix, "window_layer: bad prefix");
   const WindowScratch s(l);
   const Memory m{static_cast<char*>(scratch)};
   float* ws = m.floats(s.ws);

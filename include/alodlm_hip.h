@@ -236,8 +236,9 @@ int alodlm_norm_product(const void* x, int64_t ldx, const void* norm_weight, flo
  * written into rows [prefix, prefix + rows) of kbuf / vbuf [.., nkv*dh]; y
  * [rows, hidden].  Weights as alodlm_gemm takes them: w* [out, in], w*_t their
  * [in, out] copies or NULL; cos/sin [rows, dh].  The attention's mask
- * arguments are alodlm_attention_fwd's, its key rows start `base` rows into
- * the buffers.  scratch: alodlm_window_layer_scratch(...) bytes, 256-byte
+ * arguments are alodlm_attention_fwd's for query rows that start at the
+ * window: their row 0 is key row `base`, which must be `prefix` (cached keys lie
+ * at negative rows).  scratch: alodlm_window_layer_scratch(...) bytes, 256-byte
  * aligned. */
 int64_t alodlm_window_layer_scratch(int64_t rows, int64_t hidden, int64_t nq, int64_t nkv,
                                     int64_t dh, int64_t inter, int dtype);

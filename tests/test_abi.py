@@ -92,6 +92,23 @@ def test_no_alloc_rmsnorm_bwd_rejects_oversize_on_the_host():
                   65536, 2048, _lib.BF16_CODE, None)
 
 
+def test_window_layer_takes_query_rows_at_the_prefix_only():
+    """alodlm_window_layer's query rows start at the window, so a mask based on
+    any other key row would read keys of the wrong rows, some before the buffer:
+    rejected on the host (no rows: nothing is launched)."""
+    from alodlm_amd import _lib
+    if not _lib.LIBRARY.exists():
+        pytest.skip("library not built")
+
+    def window(prefix, base):
+        _lib.call("alodlm_window_layer", *[None] * 17, prefix, base, None, None, None, 0, 32, None,
+                  None, 0, 256, 2, 1, 128, 512, 1e-6, _lib.BF16_CODE, None)
+    for prefix, base in ((300, 256), (300, 0), (5, 6), (-1, -1)):
+        with pytest.raises(ValueError, match="prefix"):
+            window(prefix, base)
+    window(300, 300)
+
+
 def test_embed_plan_limits_on_the_host():
     """The embedding plan and scatter reject row counts of 2^24 and more (one
     256-thread workgroup per chunk) before any launch; the plan and workspace
