@@ -204,9 +204,10 @@ int alodlm_rotary_bwd(const void* dout, const void* cos_tab, const void* sin_tab
  *           ALODLM_EPI_STORE_F32 Cf32 = alpha*acc            (C is float: the first
  *                               contribution to a gradient, which then needs no zeroing)
  * workspace: float scratch of alodlm_gemm_workspace(M, N, K, epilogue, dtype)
- * floats for split-K partials of products with few output tiles (summed in
- * split order, then rounded once).  May be NULL (the
- * product then runs unsplit); unused when the query returns 0.
+ * floats for split-K partials of products with few output tiles, of any
+ * epilogue and dtype (summed in split order, then rounded once).  The sizes
+ * are this version's: query them, for every product that shares the buffer.
+ * May be NULL (the product then runs unsplit); unused when the query returns 0.
  * ------------------------------------------------------------------------ */
 enum { ALODLM_EPI_STORE = 0, ALODLM_EPI_RESIDUAL = 1, ALODLM_EPI_ACCUM = 2,
        ALODLM_EPI_STORE_F32 = 3 };

@@ -78,6 +78,21 @@ def test_gemm_workspace_policy():
     assert q(4096, 2048, 32768, ACCUM, BF16) == 4 * 4096 * 2048
 
 
+def test_workspace_sizes_belong_to_the_abi_version():
+    """Products that needed no workspace when version 7 came (bf16 residual,
+    short-K bf16 store, float32) split K when they get one: a caller that sized
+    a shared buffer by those answers must be stopped by the version."""
+    from alodlm_amd import _lib
+    if not _lib.LIBRARY.exists():
+        pytest.skip("library not built")
+    q = lambda *a: _lib.query("alodlm_gemm_workspace", *a)
+    STORE, RESIDUAL, BF16, F32 = 0, 1, 1, 0
+    grown = [(300, 2048, 6144, RESIDUAL, BF16), (300, 2048, 12288, STORE, BF16),
+             (300, 2048, 6144, STORE, F32)]
+    assert all(q(*args) > 0 for args in grown)
+    assert _lib.ABI_VERSION >= 8 and _lib.load().alodlm_abi_version() == _lib.ABI_VERSION
+
+
 def test_no_alloc_rmsnorm_bwd_rejects_oversize_on_the_host():
     """The allocation-free RMSNorm backward checks its scratch limit before
     touching the device (32768 x 2048 fits the 4 Mi-float scratch, 65536 x 2048
