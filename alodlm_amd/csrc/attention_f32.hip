@@ -17,11 +17,14 @@
 // A workgroup owns one 32-row tile of one head; its four waves take the tile's
 // key (query) tiles in turn and add up in LDS in wave order, so that a short
 // pack (the 700 rows of one 350-token segment: 352 tiles) still fills the chip.
+// A tile of rows with an infinity or NaN among the rows it multiplies is done
+// again row by row (attention_rows.h), so that no row depends on rows that the
+// mask hides from it; the check is VALU work beside the matrix instructions.
 // At that shape (16 / 8 heads): forward 603 us, dQ 635, dK/dV 1269 with one
 // wave per row and no matrix instruction.
 #include <limits.h>
 
-#include "attention_common.h"
+#include "attention_rows.h"
 
 namespace {
 
@@ -53,9 +56,11 @@ __device__ __forceinline__ f32x16_t dot_rows(const float* p, int half, const flo
 }
 
 // acc[d] += sum over the tile's rows t of p[row0 + t][4 col + d] * w[t]
-// (rows past `last` re-read it: their weights are zero).
+// (rows past `last` re-read it: their weights are zero).  z becomes NaN where a
+// row holds an infinity or NaN: the product gives it a part in the sums of
+// lanes whose weight for it is zero because the mask hides it.
 __device__ __forceinline__ void add_rows(f32x16_t (&acc)[NB], const float* p, int64_t ld, int row0,
-                                         int last, int col, int half, const f32x16_t& w) {
+                                         int last, int col, int half, const f32x16_t& w, float& z) {
 #pragma unroll
   for (int t = 0; t < 16; ++t) {
     int r = row0 + 8 * (t >> 2) + 4 * half + (t & 3);
@@ -65,7 +70,19 @@ __device__ __forceinline__ void add_rows(f32x16_t (&acc)[NB], const float* p, in
     acc[1] = mfma2(x.y, w[t], acc[1]);
     acc[2] = mfma2(x.z, w[t], acc[2]);
     acc[3] = mfma2(x.w, w[t], acc[3]);
+    z = fmaf(x.w, 0.f, fmaf(x.z, 0.f, fmaf(x.y, 0.f, fmaf(x.x, 0.f, z))));
   }
+}
+
+// Whether some wave of the workgroup met such a row.
+__device__ __forceinline__ bool any_wave(int* flags, int wave, int lane, float z) {
+  const bool mine = __any(z != 0.f);
+  if (lane == 0) flags[wave] = mine;
+  __syncthreads();
+  bool some = false;
+#pragma unroll
+  for (int v = 0; v < AW; ++v) some |= flags[v] != 0;
+  return some;
 }
 
 // This lane's intervals and their union over the wave (the tile's ranges).
@@ -136,6 +153,7 @@ attn_fwd_f32_kernel(const float* __restrict__ q, const float* __restrict__ k,
                     float* __restrict__ lse, int rows, int nq, int nkv, int64_t B, float scale) {
   __shared__ float4 lds[AW * 16 * 64];
   __shared__ float ml[2][AW][32];
+  __shared__ int flags[AW];
   const int lane = threadIdx.x & 63, half = lane >> 5, col = lane & 31;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int h = blockIdx.x, hk = h / (nq / nkv);
@@ -149,6 +167,7 @@ attn_fwd_f32_kernel(const float* __restrict__ q, const float* __restrict__ k,
   const float* vh = v + hk * HD;
   f32x16_t acc[NB] = {zero16(), zero16(), zero16(), zero16()};
   float m = -INFINITY, l = 0.f;
+  float z = 0.f;
   int turn = 0;
 #pragma unroll 1
   for (int rg = 0; rg < 2; ++rg)
@@ -180,10 +199,15 @@ attn_fwd_f32_kernel(const float* __restrict__ q, const float* __restrict__ k,
       for (int i = 0; i < NB; ++i)
 #pragma unroll
         for (int t = 0; t < 16; ++t) acc[i][t] *= corr;
-      add_rows(acc, vh, ldv, k0, last, col, half, s);
+      add_rows(acc, vh, ldv, k0, last, col, half, s, z);
     }
   if (half == 0) { ml[0][wave][col] = m; ml[1][wave][col] = l; }
-  __syncthreads();
+  if (any_wave(flags, wave, lane, z)) {  // the rows one by one, which reads allowed keys only
+    for (int r = blockIdx.y * 32 + wave; r < rows && r < (int)(blockIdx.y + 1) * 32; r += AW)
+      attn_fwd_row<float>(q, k, v, ldv, bounds, row_segment, o, lse, rows, nq, nkv, HD, B, scale, r,
+                          h);
+    return;
+  }
   float M = -INFINITY, L = 0.f, w[AW];
 #pragma unroll
   for (int i = 0; i < AW; ++i) M = fmaxf(M, ml[0][i][col]);
@@ -203,6 +227,7 @@ attn_dq_f32_kernel(const float* __restrict__ q, const float* __restrict__ k,
                    const int64_t* __restrict__ bounds, const int32_t* __restrict__ row_segment,
                    float* __restrict__ dq, int rows, int nq, int nkv, int64_t B, float scale) {
   __shared__ float4 lds[AW * 16 * 64];
+  __shared__ int flags[AW];
   const int lane = threadIdx.x & 63, half = lane >> 5, col = lane & 31;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int h = blockIdx.x, hk = h / (nq / nkv);
@@ -218,6 +243,7 @@ attn_dq_f32_kernel(const float* __restrict__ q, const float* __restrict__ k,
   const float* kh = k + hk * HD;
   const float* vh = v + hk * HD;
   f32x16_t acc[NB] = {zero16(), zero16(), zero16(), zero16()};
+  float z = 0.f;
   int turn = 0;
 #pragma unroll 1
   for (int rg = 0; rg < 2; ++rg)
@@ -234,8 +260,14 @@ attn_dq_f32_kernel(const float* __restrict__ q, const float* __restrict__ k,
         s[t] = key >= g.lo[rg] && key < g.hi[rg]
                    ? expf(s[t] * scale - ls) * (dp[t] - de) * scale : 0.f;
       }
-      add_rows(acc, kh, ldk, k0, last, col, half, s);
+      add_rows(acc, kh, ldk, k0, last, col, half, s, z);
     }
+  if (any_wave(flags, wave, lane, z)) {
+    for (int r = blockIdx.y * 32 + wave; r < rows && r < (int)(blockIdx.y + 1) * 32; r += AW)
+      attn_dq_row<float>(q, k, v, ldv, lse, delta, dout, bounds, row_segment, dq, rows, nq, nkv, HD,
+                         B, scale, r, h);
+    return;
+  }
   combine(lds, acc, nullptr, wave, lane, 1.f, dq + row * ldq + h * HD, valid);
 }
 
@@ -247,6 +279,7 @@ attn_dkdv_f32_kernel(const float* __restrict__ q, const float* __restrict__ k,
                      float* __restrict__ dk, float* __restrict__ dv, int64_t lddv, int rows,
                      int nq, int nkv, int64_t B, float scale) {
   __shared__ float4 lds[AW * 16 * 64];
+  __shared__ int flags[AW];
   const int lane = threadIdx.x & 63, half = lane >> 5, col = lane & 31;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int hk = blockIdx.x, group = nq / nkv;
@@ -260,6 +293,7 @@ attn_dkdv_f32_kernel(const float* __restrict__ q, const float* __restrict__ k,
   row_frags(v + rr * ldv + hk * HD, half, vf);
   f32x16_t dka[NB] = {zero16(), zero16(), zero16(), zero16()};
   f32x16_t dva[NB] = {zero16(), zero16(), zero16(), zero16()};
+  float z = 0.f;
   int turn = 0;
 #pragma unroll 1
   for (int h = hk * group; h < (hk + 1) * group; ++h) {
@@ -282,9 +316,15 @@ attn_dkdv_f32_kernel(const float* __restrict__ q, const float* __restrict__ k,
           p[t] = in ? expf(p[t] * scale - lse[at]) : 0.f;
           ds[t] = in ? p[t] * (ds[t] - delta[at]) * scale : 0.f;
         }
-        add_rows(dva, dh, ldq, q0, last, col, half, p);
-        add_rows(dka, qh, ldq, q0, last, col, half, ds);
+        add_rows(dva, dh, ldq, q0, last, col, half, p, z);
+        add_rows(dka, qh, ldq, q0, last, col, half, ds, z);
       }
+  }
+  if (any_wave(flags, wave, lane, z)) {
+    for (int r = blockIdx.y * 32 + wave; r < rows && r < (int)(blockIdx.y + 1) * 32; r += AW)
+      attn_dkdv_row<float>(q, k, v, ldv, lse, delta, dout, bounds, row_segment, dk, dv, lddv, rows,
+                           nq, nkv, HD, B, scale, r, hk);
+    return;
   }
   combine(lds, dka, nullptr, wave, lane, 1.f, dk + row * ldk + hk * HD, valid);
   __syncthreads();

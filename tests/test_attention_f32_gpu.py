@@ -75,3 +75,59 @@ def test_window(prefix, window):
            nq, nkv, DH, 32, L.F32_CODE, torch.cuda.current_stream().cuda_stream)
     allowed = torch.arange(prefix + window) <= torch.arange(prefix, prefix + window)[:, None]
     _close(o, _reference(q.double(), k.double(), v.double(), allowed))
+
+
+@pytest.mark.parametrize("which", ["q", "k", "v", "do"])
+@pytest.mark.parametrize("value", [float("nan"), float("inf")])
+def test_hidden_rows_take_no_part(which, value):
+    """A row holding a NaN or infinity reaches only the rows that the mask lets
+    see it: the outputs and query gradients of the other queries, and the key
+    and value gradients of keys none of the reached queries sees, are those of
+    a pack without it (within the float32 bound: the affected tiles are summed
+    row by row).  Segments of one 32-row tile share it."""
+    log(f"f32 attention with {value} in {which}")
+    offsets, nq, nkv = [0, 33, 38, 102], 4, 2
+    N = 2 * offsets[-1]
+    g = torch.Generator().manual_seed(5)
+    t = {n: torch.randn(N, h, DH, generator=g) for n, h in
+         (("q", nq), ("k", nkv), ("v", nkv), ("do", nq))}
+    plan = sparse_plan([2 * o for o in offsets], 8, "sdpa")
+    allowed = DualStreamMask(offsets, 8, DEV).dense().cpu()
+
+    def run(t):
+        leaves = [t[n].to(DEV).requires_grad_(True) for n in ("q", "k", "v")]
+        out = sparse_attention(*leaves, plan)
+        out.backward(t["do"].to(DEV))
+        return [out.detach().cpu()] + [x.grad.cpu() for x in leaves]
+    clean = run(t)
+    for row in (12, 20, 66, 75, 150, N - 1):  # clean and noisy rows of every segment
+        bad = dict(t)
+        bad[which] = t[which].clone()
+        bad[which][row, :, 17] = value
+        reached = allowed[:, row] if which in ("k", "v") else torch.arange(N) == row
+        keys = ~allowed[reached].any(0)
+        assert bool((~reached).any()) and bool(keys.any())
+        for got, ref, rows in zip(run(bad), clean, (~reached, ~reached, keys, keys)):
+            assert bool(got[rows].isfinite().all()), (row, value)
+            _close(got[rows], ref[rows].double())
+
+
+def test_window_rows_before_a_bad_one():
+    """A window row whose value is not finite leaves the rows before it alone."""
+    log("f32 attention window with infinite later rows")
+    nq, nkv, prefix, window = 4, 2, 21, 24
+    g = torch.Generator().manual_seed(9)
+    q = torch.randn(window, nq, DH, generator=g)
+    k, v = (torch.randn(prefix + window, nkv, DH, generator=g) for _ in range(2))
+    allowed = torch.arange(prefix + window) <= torch.arange(prefix, prefix + window)[:, None]
+    ref = _reference(q.double(), k.double(), v.double(), allowed)
+    v[prefix + 10] = float("inf")
+    mask = WindowMask(prefix, window, False, DEV, block_size=32)
+    qd, kd, vd = q.to(DEV), k.to(DEV), v.to(DEV)
+    o, lse = torch.empty_like(qd), torch.empty(nq, window, device=DEV)
+    shift = mask.base * nkv * DH * 4
+    L.call("alodlm_attention_fwd", L.ptr(qd), L.ptr(kd) + shift, L.ptr(vd) + shift, nkv * DH,
+           L.ptr(mask.boundaries), L.ptr(mask.row_segment), None, 0, L.ptr(o), L.ptr(lse), window,
+           nq, nkv, DH, 32, L.F32_CODE, torch.cuda.current_stream().cuda_stream)
+    _close(o[:10], ref[:10])
+    assert not bool(o[10:].isfinite().any())
