@@ -330,8 +330,8 @@ class Kernels:
         need = query("alodlm_gemm_workspace", M, N, K, epi, self.code)
         if need:
             ws = self._workspace(need)
-        call("alodlm_gemm_chain" if chain else "alodlm_gemm", ptr(A), lda, a_k, ptr(B), ldb, b_k, ptr(C), ldc, ptr(R), ldr, M, N, K,
-             alpha, epi, self.code, ptr(ws), self._stream())
+        call("alodlm_gemm_chain" if chain else "alodlm_gemm", ptr(A), lda, a_k, ptr(B), ldb, b_k,
+             ptr(C), ldc, ptr(R), ldr, M, N, K, alpha, epi, self.code, ptr(ws), self._stream())
 
     def _product(self, x, ldx, w, w_t, y, M, N, K, epi=EPI_STORE, R=None, ldr=0):
         """y = x . w^T (+ R) with w [N, K]: through the out-contiguous copy w_t
@@ -638,22 +638,31 @@ class _LayerFunction(torch.autograd.Function):
         kernels, w, d = ctx.kernels, ctx.w, ctx.kernels.dims
         H, W, I, QD = d.hidden, d.qkv_width, d.intermediate, d.heads * d.head_dim
         # the matrices' gradients in the parameter dtype, written by their
-        # products; the norm weights' sums in float32
-        mats = kernels._empty(W * H + H * QD + 3 * I * H).split([W * H, H * QD, 2 * I * H, H * I])
+        # products (q|k|v and gate|up by one each); the norm weights' sums in
+        # float32
+        qd, kd = QD, d.kv_heads * d.head_dim
         norms = torch.zeros(2 * H + 2 * d.head_dim, dtype=torch.float32, device=kernels.device)
-        gw = LayerGrads(mats[0].view(W, H), mats[1].view(H, QD), mats[2].view(2 * I, H),
-                        mats[3].view(H, I), *norms.split([H, H, d.head_dim, d.head_dim]),
+        gw = LayerGrads(kernels._empty(W, H), kernels._empty(H, QD), kernels._empty(2 * I, H),
+                        kernels._empty(H, I), *norms.split([H, H, d.head_dim, d.head_dim]),
                         stored=True)
         x, k, saved = ctx.saved
         dx = kernels.layer_call_bwd(dy.contiguous(), x, k, saved, w, gw, ctx.rope, ctx.mask,
                                     ctx.chain)
         ctx.saved = None
+        needed = ctx.needs_input_grad[5:]
+
+        def members(rows, sizes, needs):
+            # views of the group's buffer while all of it is wanted, else copies:
+            # one gradient does not hold the others' memory
+            views = rows.split(sizes)
+            return views if all(needs) else [v.clone() if n else None for v, n in zip(views, needs)]
         if len({dtype for _, dtype in ctx.shapes[7:]}) == 1:  # one cast for the four
             norms = norms.to(ctx.shapes[7][1])
-        qd, kd = QD, d.kv_heads * d.head_dim
-        parts = [gw.wqkv[:qd], gw.wqkv[qd:qd + kd], gw.wqkv[qd + kd:], gw.wo, gw.wgu[:I],
-                 gw.wgu[I:], gw.wd, *norms.split([H, H, d.head_dim, d.head_dim])]
-        grads = [g.view(shape).to(dtype) for g, (shape, dtype) in zip(parts, ctx.shapes)]
+        parts = [*members(gw.wqkv, [qd, kd, kd], needed[:3]), gw.wo,
+                 *members(gw.wgu, [I, I], needed[4:6]), gw.wd,
+                 *norms.split([H, H, d.head_dim, d.head_dim])]
+        grads = [g.view(shape).to(dtype) if n else None
+                 for g, n, (shape, dtype) in zip(parts, needed, ctx.shapes)]
         return (None, None, None, None, dx, *grads)
 
 

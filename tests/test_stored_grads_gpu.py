@@ -10,7 +10,8 @@ import torch
 
 from alodlm_amd import _lib as L
 from alodlm_amd.engine import Dims
-from alodlm_amd.layers import DualStreamMask, Kernels, LayerGrads, LayerWeights, Rope
+from alodlm_amd.layers import (DualStreamMask, Kernels, LayerGrads, LayerWeights, Rope,
+                               _LayerFunction)
 from tests.helpers import log
 
 pytestmark = pytest.mark.gpu
@@ -80,3 +81,41 @@ def test_layer_gradients_stored(lengths, dtype):
         if dtype == torch.bfloat16:
             bound = bound + 2.0 ** -8 * b.abs()
         assert bool(((a.float() - b).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("trained", [(0,), (1, 4), (3, 6), tuple(range(11))])
+def test_gradients_hold_their_own_memory(trained, dtype):
+    """A parameter's gradient holds no memory of parameters that are not
+    trained: its storage is its own size, or its group's (q|k|v, gate|up: one
+    product writes them) when the whole group is trained.  Values do not depend
+    on which parameters are."""
+    log(f"gradient storage, trained parameters {trained} {dtype}")
+    H, nq, nkv, dh, I = 256, 2, 1, 128, 264
+    kernels = Kernels(Dims(H, nq, nkv, dh, I, 0, 1, 1e-6, 0.0), dtype, torch.device(DEV))
+    g = torch.Generator(device=DEV).manual_seed(7)
+    shapes = [(nq * dh, H), (nkv * dh, H), (nkv * dh, H), (H, nq * dh), (I, H), (I, H), (H, I),
+              (H,), (H,), (dh,), (dh,)]
+    mask = DualStreamMask([0, 40, 65], 32, torch.device(DEV))
+    rope = Rope(positions=torch.arange(mask.rows, device=DEV) % 40,
+                inv_freq=torch.rand(dh // 2, generator=g, device=DEV))
+    data = [0.05 * torch.randn(*s, generator=g, device=DEV) + (len(s) == 1) for s in shapes]
+    x, dy = (torch.randn(mask.rows, H, generator=g, device=DEV).to(dtype) for _ in range(2))
+
+    def grads(which):
+        params = [t.to(dtype, copy=True).requires_grad_(i in which) for i, t in enumerate(data)]
+        _LayerFunction.apply(kernels, mask, rope, False, x, *params)[0].backward(dy)
+        return [p.grad for p in params]
+    full, got = grads(range(11)), grads(trained)
+    groups = ((0, 1, 2), (3,), (4, 5), (6,))
+    for i, t in enumerate(got):
+        assert (t is not None) == (i in trained)
+        if t is None:
+            continue
+        assert torch.equal(t, full[i]), i
+        if i < 7:
+            group = next(m for m in groups if i in m)
+            owners = group if set(group) <= set(trained) else (i,)
+            size = sum(data[j].numel() for j in owners) * t.element_size()
+            held = t.untyped_storage().nbytes()
+            assert held == size, i
