@@ -61,3 +61,22 @@ def test_products(M, N, K, ak, bk, epi):
                torch.cuda.current_stream().cuda_stream)
         err = (out.double() - ref).abs()
         assert bool((err <= bound + 1e-6).all()), float((err - bound).max())
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("epi", [0, 1, 2, 3])
+@pytest.mark.parametrize("ak,bk", [(0, 0), (1, 1)])
+def test_empty_sum(epi, ak, bk, dtype):
+    """K = 0 (the weight gradient of no rows): zeros are stored, the residual is
+    copied, an accumulated output stays."""
+    log(f"gemm K=0 ak={ak} bk={bk} epi={epi} {dtype}")
+    M, N = 264, 136
+    f32 = epi in (L.EPI_ACCUM, L.EPI_STORE_F32)
+    C = torch.randn(M, N, device=DEV).to(torch.float32 if f32 else dtype)
+    R, before = torch.randn(M, N, device=DEV).to(dtype), C.clone()
+    A, B = torch.zeros(8, device=DEV, dtype=dtype), torch.zeros(8, device=DEV, dtype=dtype)
+    L.call("alodlm_gemm", L.ptr(A), 8 if ak else M, ak, L.ptr(B), 8 if bk else N, bk, L.ptr(C), N,
+           L.ptr(R), N, M, N, 0, 1.0, epi, L.dtype_code(dtype), None,
+           torch.cuda.current_stream().cuda_stream)
+    want = R if epi == L.EPI_RESIDUAL else before if epi == L.EPI_ACCUM else torch.zeros_like(C)
+    assert torch.equal(C, want)

@@ -60,3 +60,26 @@ def test_layer_call_matches_steps(H, nq, nkv, dh, I, lengths, block, tables, dty
         assert torch.equal(v.view(N, KD), save[0][3][:, QD + KD:])
     for name in ("wqkv", "wo", "wgu", "wd", "ln1", "ln2", "qn", "kn"):
         assert torch.equal(getattr(got, name), getattr(ref, name)), name
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_layer_call_of_no_rows(dtype):
+    """No rows: empty outputs, zero weight gradients."""
+    log(f"layer call of no rows {dtype}")
+    H, nq, nkv, dh, I = 256, 2, 1, 128, 264
+    kernels = Kernels(Dims(H, nq, nkv, dh, I, 0, 1, 1e-6, 0.0), dtype, torch.device(DEV))
+    W, QD = kernels.dims.qkv_width, nq * dh
+    shapes = ((W, H), (H, QD), (2 * I, H), (H, I))
+    w = LayerWeights(*[torch.ones(s, device=DEV).to(dtype) for s in shapes],
+                     *[torch.ones(n, device=DEV).to(dtype) for n in (H, H, dh, dh)])
+    mask = DualStreamMask([0, 0], 32, torch.device(DEV))
+    rope = Rope(cos=torch.empty(0, dh, dtype=dtype, device=DEV),
+                sin=torch.empty(0, dh, dtype=dtype, device=DEV))
+    x = torch.empty(0, H, dtype=dtype, device=DEV)
+    g = LayerGrads(*[torch.full(s, float("nan"), dtype=dtype, device=DEV) for s in shapes],
+                   *[torch.zeros(n, device=DEV) for n in (H, H, dh, dh)], stored=True)
+    y, k, v, saved = kernels.layer_call_fwd(w, x, rope, mask)
+    dx = kernels.layer_call_bwd(x, x, k, saved, w, g, rope, mask)
+    assert y.shape == dx.shape == (0, H) and k.shape == v.shape == (0, nkv, dh)
+    for t in (g.wqkv, g.wo, g.wgu, g.wd, g.ln1, g.ln2, g.qn, g.kn):
+        assert not bool(t.any())
