@@ -12,6 +12,7 @@ import torch
 
 LIBRARY = Path(__file__).resolve().parent / "libalodlm_hip.so"
 ABI_VERSION = 8
+FEW_ROWS = 64  # ALODLM_FEW_ROWS
 
 P = ctypes.c_void_p
 I64 = ctypes.c_int64

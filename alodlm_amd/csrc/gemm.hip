@@ -4,17 +4,20 @@
 //
 // bf16: few rows go to gemm_skinny.hip, the rest to the 256x256 tiles of
 // gemm_dl.hip or the 128-column tiles of gemm_mid.hip (bf16_plan, below).  What
-// none of them takes (unaligned operands, small float outputs) runs in
-// gemm_big.hip or on the tiles of this file: 128x128x64, 4 wavefronts in a 2x2
-// grid, each computing a 64x64 block with v_mfma_f32_32x32x16_bf16.  Operands are staged through LDS
-// in k-contiguous rows (padded by 8 elements); an operand stored m/n-contiguous
-// ([K, M] in memory, as in the backward's dW and dX products) is transposed
-// while it is staged: each thread loads an 8(k) x 4(m) block with 8-byte
-// loads and writes four 16-byte k-rows.  Global loads for tile k+1 are issued
-// before the MFMAs of tile k (register prefetch, double-buffered LDS).
+// none of them takes - K a multiple of 8 but not of 32 with a k-contiguous
+// operand, m/n-contiguous ones of no whole 8 rows, fewer than 8 rows or columns,
+// operands of 2 GiB and more whose K is no multiple of 32 - runs in gemm_big.hip
+// or on the tiles of this file: 128x128x64, 4 wavefronts in a 2x2 grid, each
+// computing a 64x64 block with v_mfma_f32_32x32x16_bf16.  Operands are staged
+// through LDS in k-contiguous rows (padded by 8 elements); an operand stored
+// m/n-contiguous ([K, M] in memory, as in the backward's dW and dX products) is
+// transposed while it is staged: each thread loads an 8(k) x 4(m) block with
+// 8-byte loads and writes four 16-byte k-rows.  Global loads for tile k+1 are
+// issued before the MFMAs of tile k (register prefetch, double-buffered LDS).
 //
-// float: gemm_skinny.hip (few rows) and gemm_f32.hip; unaligned operands: a
-// plain LDS-tiled FMA kernel.
+// float: gemm_skinny.hip (few rows) and gemm_f32.hip.  Operands that are not
+// 16-byte aligned (pointers or row strides), of either type: a plain LDS-tiled
+// FMA kernel.
 #include <type_traits>
 
 #include "common.h"

@@ -26,29 +26,11 @@
 typedef __attribute__((__vector_size__(8 * sizeof(short)))) short bf16x8_t;
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float f32x4_t;
 typedef short v4s_t __attribute__((ext_vector_type(4)));
-typedef int v4i_t __attribute__((ext_vector_type(4)));
 #define LDS_AS __attribute__((address_space(3)))
 
 namespace {
 
 constexpr int TN = 128, KD = 32, NW = 4;
-
-// 16 bytes per lane from the buffer's byte voff + soff (zeros past its end)
-// into the 16-byte slot `lane` of the LDS byte address m0v.
-__device__ __forceinline__ void dma16_buf(v4i_t rsrc, uint32_t voff, uint32_t soff, uint32_t m0v) {
-  asm volatile("buffer_load_dwordx4 %0, %1, %2 offen lds"
-               ::"v"(voff), "s"(rsrc), "s"(soff), "{m0}"(m0v) : "memory");
-}
-
-__device__ __forceinline__ v4i_t buffer_of(const bf16_t* p, int64_t bytes) {
-  const uint64_t b = (uint64_t)(uintptr_t)p;
-  v4i_t r;
-  r.x = __builtin_amdgcn_readfirstlane((int)(uint32_t)b);
-  r.y = __builtin_amdgcn_readfirstlane((int)(uint32_t)(b >> 32));
-  r.z = __builtin_amdgcn_readfirstlane((int)(uint32_t)bytes);
-  r.w = 0x00020000;
-  return r;
-}
 
 // One operand: this wave's lane offsets into the buffer, the byte step from one
 // k stage to the next, and the lane's fragment offsets within a stage.

@@ -3,7 +3,7 @@
 
 #include "common.h"
 
-constexpr int64_t SKINNY_M = 64;  // rows up to which it is taken
+constexpr int64_t SKINNY_M = ALODLM_FEW_ROWS;  // rows up to which it is taken
 
 bool gemm_skinny_eligible(const void* A, int64_t lda, int a_kmajor, const void* B, int64_t ldb,
                           int b_kmajor, int64_t M, int64_t N, int64_t K, int epi, int dtype);

@@ -69,26 +69,6 @@ __device__ __forceinline__ uint4 normed(uint4 x, uint4 w, float r) {
 // second half as up projection and stores silu(gate) * up (N / 2 columns).
 constexpr int SKINNY_NORM = 1, SKINNY_GLU = 2;
 
-typedef int v4i_t __attribute__((ext_vector_type(4)));
-
-// 16 (4) bytes per lane from the buffer's byte voff (zeros past its end) into
-// the lane's slot after the LDS byte address m0v.
-__device__ __forceinline__ void dma16_buf(v4i_t rsrc, uint32_t voff, uint32_t m0v) {
-  asm volatile("buffer_load_dwordx4 %0, %1, 0 offen lds" ::"v"(voff), "s"(rsrc), "{m0}"(m0v) : "memory");
-}
-__device__ __forceinline__ void dma4_buf(v4i_t rsrc, uint32_t voff, uint32_t m0v) {
-  asm volatile("buffer_load_dword %0, %1, 0 offen lds" ::"v"(voff), "s"(rsrc), "{m0}"(m0v) : "memory");
-}
-__device__ __forceinline__ v4i_t buffer_of(const void* p, int64_t bytes) {
-  const uint64_t b = (uint64_t)(uintptr_t)p;
-  v4i_t r;
-  r.x = __builtin_amdgcn_readfirstlane((int)(uint32_t)b);
-  r.y = __builtin_amdgcn_readfirstlane((int)(uint32_t)(b >> 32));
-  r.z = __builtin_amdgcn_readfirstlane((int)(uint32_t)bytes);
-  r.w = 0x00020000;
-  return r;
-}
-
 // MT: 16-row blocks of A; NT: 16-row blocks of W per workgroup; H: fragments
 // (64 bytes of a row) per stage; S: stages of a wave's ring.
 template <typename T, int MT, int NT, int H, int S, int EPI, int FUSE = 0>

@@ -5,7 +5,8 @@
 // steps share.  16 window rows keep the chip busy for 57 us per layer, and the
 // separate calls with their output allocations took 95 us of host time, 36 us
 // now.  Forward and backward of a 1.7B layer over 300 rows: 530 us a call and
-// 440 now, with about 400 us of kernels; 2474 rows 1213 and 1199.
+// about 450 now (440 to 458 from card to card), with about 400 us of kernels;
+// 2474 rows 1213 and 1199.
 #include <algorithm>
 
 #include "attention.h"
@@ -14,7 +15,6 @@
 namespace {
 
 constexpr int64_t FUSED_ROWS = 16;   // alodlm_norm_product's rows
-constexpr int64_t SKINNY_ROWS = 64;  // rows up to which products stream [out, in] weights
 
 #define RUN(call)           \
   do {                      \
@@ -40,7 +40,7 @@ struct Layer {
   // C = A w^T (+ R), w [N, K] or its copy w_t [K, N] where that serves the rows
   int product(const void* A, const void* w, const void* w_t, void* C, int64_t N, int64_t K,
               const void* R, float* ws) const {
-    const bool copy = w_t != nullptr && rows > SKINNY_ROWS;
+    const bool copy = w_t != nullptr && rows > ALODLM_FEW_ROWS;
     return (chain ? alodlm_gemm_chain : alodlm_gemm)(
         A, K, 1, copy ? w_t : w, copy ? N : K, copy ? 0 : 1, C, N, R, R ? N : 0, rows, N, K, 1.f,
         R ? ALODLM_EPI_RESIDUAL : ALODLM_EPI_STORE, dtype, ws, stream);

@@ -9,7 +9,8 @@
 // prefetch.  Kernels using these helpers therefore wait for their own loads
 // explicitly (s_waitcnt vmcnt(n) before the barrier that publishes a tile).
 // Loads the compiler does not count only make its own vmcnt waits more
-// conservative, never less.  M0 is saved and restored around each load.
+// conservative, never less.  M0 is saved and restored around each global load;
+// the buffer loads name it as an input.
 #pragma once
 
 #include <stdint.h>
@@ -82,4 +83,30 @@ __device__ __forceinline__ void dma4_v(const void* g, uint32_t lds) {
       : "=&s"(saved)
       : "v"(g), "s"(lds)
       : "memory");
+}
+
+// A buffer of `bytes` bytes at p (wave-uniform) for the loads below, whose range
+// check returns zeros past its end.
+typedef int v4i_t __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ v4i_t buffer_of(const void* p, int64_t bytes) {
+  const uint64_t b = (uint64_t)(uintptr_t)p;
+  v4i_t r;
+  r.x = __builtin_amdgcn_readfirstlane((int)(uint32_t)b);
+  r.y = __builtin_amdgcn_readfirstlane((int)(uint32_t)(b >> 32));
+  r.z = __builtin_amdgcn_readfirstlane((int)(uint32_t)bytes);
+  r.w = 0x00020000;
+  return r;
+}
+
+// 16 (4) bytes per lane from the buffer's byte voff (+ soff) into the lane's slot
+// after the LDS byte address m0v.
+__device__ __forceinline__ void dma16_buf(v4i_t rsrc, uint32_t voff, uint32_t soff, uint32_t m0v) {
+  asm volatile("buffer_load_dwordx4 %0, %1, %2 offen lds"
+               ::"v"(voff), "s"(rsrc), "s"(soff), "{m0}"(m0v) : "memory");
+}
+__device__ __forceinline__ void dma16_buf(v4i_t rsrc, uint32_t voff, uint32_t m0v) {
+  asm volatile("buffer_load_dwordx4 %0, %1, 0 offen lds" ::"v"(voff), "s"(rsrc), "{m0}"(m0v) : "memory");
+}
+__device__ __forceinline__ void dma4_buf(v4i_t rsrc, uint32_t voff, uint32_t m0v) {
+  asm volatile("buffer_load_dword %0, %1, 0 offen lds" ::"v"(voff), "s"(rsrc), "{m0}"(m0v) : "memory");
 }

@@ -271,12 +271,10 @@ qknorm_rope128_fwd_kernel(const bf16_t* __restrict__ qkv, const bf16_t* __restri
       }
       continue;  // the head's 8 lanes together
     }
-    const bool live = true;
     const bool is_q = head < nq;
     float xa[8], xb[8];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) xa[e] = xb[e] = 0.f;
-    if (live) { Vec8<bf16_t>::load(src + head * 128 + i0, xa); Vec8<bf16_t>::load(src + head * 128 + i0 + 64, xb); }
+    Vec8<bf16_t>::load(src + head * 128 + i0, xa);
+    Vec8<bf16_t>::load(src + head * 128 + i0 + 64, xb);
     float ss = 0.f;
 #pragma unroll
     for (int e = 0; e < 8; ++e) ss += xa[e] * xa[e] + xb[e] * xb[e];
@@ -290,11 +288,9 @@ qknorm_rope128_fwd_kernel(const bf16_t* __restrict__ qkv, const bf16_t* __restri
       oa[e] = round_bf16(a * cs[e]) + round_bf16(-b * sn[e]);
       ob[e] = round_bf16(b * cb[e]) + round_bf16(a * sb[e]);
     }
-    if (live) {
-      bf16_t* dst = is_q ? q_out + (row * nq + head) * 128 : k_out + (row * nkv + head - nq) * 128;
-      Vec8<bf16_t>::store(dst + i0, oa);
-      Vec8<bf16_t>::store(dst + i0 + 64, ob);
-    }
+    bf16_t* dst = is_q ? q_out + (row * nq + head) * 128 : k_out + (row * nkv + head - nq) * 128;
+    Vec8<bf16_t>::store(dst + i0, oa);
+    Vec8<bf16_t>::store(dst + i0 + 64, ob);
   }
 }
 

@@ -30,10 +30,10 @@ import numpy as np
 import torch
 
 from . import _lib
-from ._lib import EPI_ACCUM, EPI_RESIDUAL, EPI_STORE, EPI_STORE_F32, call, ptr, query
+from ._lib import (EPI_ACCUM, EPI_RESIDUAL, EPI_STORE, EPI_STORE_F32, FEW_ROWS, call, ptr,
+                   query)
 
 TILE_ROWS = 128
-SKINNY_ROWS = 64  # rows up to which a product streams its [out, in] weight
 
 
 def allowed_pairs(length, block_size):
@@ -190,15 +190,14 @@ class WindowMask:
     Segment row r is query-buffer row r - P and key/value row r (the
     key/value pointers are offset by ``base`` = P rows, so the cached keys lie
     at negative rows); with ``tiled`` the MFMA kernels' query tiles start at
-    row P."""
+    row P.  ``q_rows`` (= W) and ``q_off`` (= 0) describe the query buffer to
+    callers that lay it out themselves."""
 
     def __init__(self, prefix, window, tiled, device, block_size=1):
         self.prefix, self.window = prefix, window
         L = prefix + window
         self.block_size = block_size
-        self.base = prefix
-        self.q_rows = L - self.base
-        self.q_off = prefix - self.base
+        self.base, self.q_rows, self.q_off = prefix, window, 0
         self.boundaries = torch.tensor([-self.base, 2 * L - self.base], dtype=torch.int64,
                                        device=device)
         self.row_segment = torch.zeros(self.q_rows, dtype=torch.int32, device=device)
@@ -277,7 +276,10 @@ def _stack_rows(*ts):
 class LayerGrads:
     """Gradient views of one layer (same layout as LayerWeights), float32; with
     ``stored`` the four projection matrices' are in the storage dtype and
-    written once (one product, rounded once) instead of accumulated."""
+    written once (one product, rounded once) instead of accumulated: what
+    ``layer_call_bwd`` takes.  (The step accumulates; ``layer_bwd`` knows both
+    so that the native call can be compared with it launch by launch, as
+    ``layer_fwd`` and ``layer_bwd`` know rotary tables.)"""
 
     def __init__(self, wqkv, wo, wgu, wd, ln1, ln2, qn, kn, stored=False):
         self.stored = stored
@@ -337,7 +339,7 @@ class Kernels:
         """y = x . w^T (+ R) with w [N, K]: through the out-contiguous copy w_t
         [K, N] when there is one and M rows fill the wide tiles it serves
         (fewer rows stream w itself, whose rows are k-contiguous)."""
-        if w_t is not None and M > SKINNY_ROWS:
+        if w_t is not None and M > FEW_ROWS:
             self._gemm(x, ldx, 1, w_t, N, 0, y, N, M, N, K, epi=epi, R=R, ldr=ldr)
         else:
             self._gemm(x, ldx, 1, w, K, 1, y, N, M, N, K, epi=epi, R=R, ldr=ldr)

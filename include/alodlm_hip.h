@@ -209,6 +209,9 @@ int alodlm_rotary_bwd(const void* dout, const void* cos_tab, const void* sin_tab
  * are this version's: query them, for every product that shares the buffer.
  * May be NULL (the product then runs unsplit); unused when the query returns 0.
  * ------------------------------------------------------------------------ */
+/* Rows up to which a product streams an [out, in] weight's k-contiguous rows;
+ * above, the wide tiles read its [in, out] copy where there is one. */
+#define ALODLM_FEW_ROWS 64
 enum { ALODLM_EPI_STORE = 0, ALODLM_EPI_RESIDUAL = 1, ALODLM_EPI_ACCUM = 2,
        ALODLM_EPI_STORE_F32 = 3 };
 int64_t alodlm_gemm_workspace(int64_t M, int64_t N, int64_t K, int epilogue, int dtype);
@@ -576,7 +579,8 @@ int alodlm_sequence_score(const float* credit, const float* logq, const int64_t*
 /* Next-token targets of autoregressive_loss (alodlm/loss.py:12-32) over the
  * dual-stream rows: clean row start + i of a segment [start, end) with
  * L = (end - start) / 2 >= 2 and i < L - 1 predicts labels[start/2 + 1 + i];
- * every other row and ignored labels (-100) get -1. */
+ * every other row and ignored labels (-100) get -1.  Kept for callers that want
+ * a target per row; autoregressive_loss itself takes alodlm_ar_rows. */
 int alodlm_ar_targets(const int64_t* labels, const int64_t* bounds, int64_t n_segments,
                       int64_t rows, int32_t* target, void* stream);
 /* The rows with a target in order: sel, target [rows] hold count[0] entries. */

@@ -93,6 +93,13 @@ def test_workspace_sizes_belong_to_the_abi_version():
     assert _lib.ABI_VERSION >= 8 and _lib.load().alodlm_abi_version() == _lib.ABI_VERSION
 
 
+def test_shared_constants_match_header():
+    from alodlm_amd import _lib
+    defines = dict(re.findall(r"#define (ALODLM_\w+) (\d+)", HEADER.read_text()))
+    assert int(defines["ALODLM_ABI_VERSION"]) == _lib.ABI_VERSION
+    assert int(defines["ALODLM_FEW_ROWS"]) == _lib.FEW_ROWS
+
+
 def test_no_alloc_rmsnorm_bwd_rejects_oversize_on_the_host():
     """The allocation-free RMSNorm backward checks its scratch limit before
     touching the device (32768 x 2048 fits the 4 Mi-float scratch, 65536 x 2048
