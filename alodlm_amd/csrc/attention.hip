@@ -187,6 +187,16 @@ extern "C" int alodlm_attention_fwd(const void* q, const void* k, const void* v,
                        block_size, dtype, false, stream);
 }
 
+extern "C" int alodlm_attention_fwd_chain(const void* q, const void* k, const void* v, int64_t ldv,
+                                          const int64_t* bounds, const int32_t* row_segment,
+                                          const int32_t* tiles, int64_t n_tiles, void* o,
+                                          float* lse, int64_t rows, int64_t nq, int64_t nkv,
+                                          int64_t dh, int64_t block_size, int dtype,
+                                          void* stream) {
+  return attention_fwd(q, k, v, ldv, bounds, row_segment, tiles, n_tiles, o, lse, rows, nq, nkv, dh,
+                       block_size, dtype, true, stream);
+}
+
 int64_t fa128_bwd_workspace(int64_t N, int nq, int nkv, int64_t n_tiles, int64_t ds_blocks);
 
 // 32x32 dS blocks per query head that the mask allows in a pack (the stored-dS

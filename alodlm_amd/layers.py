@@ -335,18 +335,18 @@ class Kernels:
         call("alodlm_gemm_chain" if chain else "alodlm_gemm", ptr(A), lda, a_k, ptr(B), ldb, b_k,
              ptr(C), ldc, ptr(R), ldr, M, N, K, alpha, epi, self.code, ptr(ws), self._stream())
 
-    def _product(self, x, ldx, w, w_t, y, M, N, K, epi=EPI_STORE, R=None, ldr=0):
+    def _product(self, x, ldx, w, w_t, y, M, N, K, epi=EPI_STORE, R=None, ldr=0, chain=False):
         """y = x . w^T (+ R) with w [N, K]: through the out-contiguous copy w_t
         [K, N] when there is one and M rows fill the wide tiles it serves
         (fewer rows stream w itself, whose rows are k-contiguous)."""
         if w_t is not None and M > FEW_ROWS:
-            self._gemm(x, ldx, 1, w_t, N, 0, y, N, M, N, K, epi=epi, R=R, ldr=ldr)
+            self._gemm(x, ldx, 1, w_t, N, 0, y, N, M, N, K, epi=epi, R=R, ldr=ldr, chain=chain)
         else:
-            self._gemm(x, ldx, 1, w, K, 1, y, N, M, N, K, epi=epi, R=R, ldr=ldr)
+            self._gemm(x, ldx, 1, w, K, 1, y, N, M, N, K, epi=epi, R=R, ldr=ldr, chain=chain)
 
-    def _attention_fwd(self, q, k, v, ldv, o, lse, mask):
+    def _attention_fwd(self, q, k, v, ldv, o, lse, mask, chain=False):
         d = self.dims
-        call("alodlm_attention_fwd", ptr(q), ptr(k), ptr(v), ldv, ptr(mask.boundaries),
+        call("alodlm_attention_fwd_chain" if chain else "alodlm_attention_fwd", ptr(q), ptr(k), ptr(v), ldv, ptr(mask.boundaries),
              ptr(mask.row_segment), ptr(mask.tiles),
              0 if mask.tiles is None else mask.tiles.shape[0], ptr(o), ptr(lse), q.shape[0],
              d.heads, d.kv_heads, d.head_dim, mask.block_size, self.code, self._stream())
@@ -362,7 +362,7 @@ class Kernels:
              ptr(dk), ptr(dv), lddv, ptr(ws), ptr(getattr(mask, "ds_base", None)), ds_blocks,
              N, d.heads, d.kv_heads, d.head_dim, mask.block_size, self.code, self._stream())
 
-    def _attention_fwd_flops(self, q, k, v, ldv, o, lse, mask):
+    def _attention_fwd_flops(self, q, k, v, ldv, o, lse, mask, chain=False):
         """Algorithmic forward FLOPs: 4*dh per allowed (q, k) pair and head."""
         return 4.0 * self.dims.head_dim * self.dims.heads * mask.pairs
 
@@ -395,7 +395,7 @@ class Kernels:
                  ptr(ws), N, d.heads, d.kv_heads, d.head_dim, d.eps, self.code, self._stream())
 
     # ------------------------------------------------------------------ layer
-    def layer_fwd(self, w, x, mask, rope, save=None, keep=(False, False), tag=None):
+    def layer_fwd(self, w, x, mask, rope, save=None, keep=(False, False), tag=None, chain=False):
         """One layer application (alodlm/model.py:49-76) over x [N, H].
 
         With ``save`` (a list) the activations the backward needs are
@@ -403,7 +403,9 @@ class Kernels:
         attention output and log-sum-exp, the post-attention residual and the
         gate|up projections; ``keep`` = (rotary q/k, norm outputs) also keeps
         those (else the backward recomputes them).  Returns y [N, H]; with
-        ``keep[0]`` the rotated q/k stay in the saved tuple (indices 9, 10)."""
+        ``keep[0]`` the rotated q/k stay in the saved tuple (indices 9, 10).
+        With ``chain`` a bf16 row's sums run in one order whatever the other
+        rows."""
         d, N, st, c = self.dims, x.shape[0], self._stream(), self.code
         H, W, I = d.hidden, d.qkv_width, d.intermediate
         QD = d.heads * d.head_dim
@@ -411,7 +413,7 @@ class Kernels:
         rstd1 = self._empty(N, dtype=torch.float32)
         call("alodlm_rmsnorm_fwd", ptr(x), ptr(w.ln1), ptr(h1), ptr(rstd1), N, H, d.eps, c, st)
         qkv = self._empty(N, W)
-        self._product(h1, H, w.wqkv, w.wqkv_t, qkv, N, W, H)
+        self._product(h1, H, w.wqkv, w.wqkv_t, qkv, N, W, H, chain=chain)
         keep_rot, keep_norm = keep if save is not None else (False, False)
         if not keep_norm:
             h1 = None
@@ -421,34 +423,35 @@ class Kernels:
         o = self._empty(N, QD)
         lse = self._empty(d.heads, N, dtype=torch.float32)
         v = qkv[:, QD + d.kv_heads * d.head_dim:]
-        self._attention_fwd(q, k, v, W, o, lse, mask)
+        self._attention_fwd(q, k, v, W, o, lse, mask, chain=chain)
         if not keep_rot:
             q = k = None
         x1 = self._empty(N, H)
-        self._product(o, QD, w.wo, w.wo_t, x1, N, H, QD, epi=EPI_RESIDUAL, R=x, ldr=H)
+        self._product(o, QD, w.wo, w.wo_t, x1, N, H, QD, epi=EPI_RESIDUAL, R=x, ldr=H, chain=chain)
         h2 = self._empty(N, H)
         rstd2 = self._empty(N, dtype=torch.float32)
         call("alodlm_rmsnorm_fwd", ptr(x1), ptr(w.ln2), ptr(h2), ptr(rstd2), N, H, d.eps, c, st)
         gu = self._empty(N, 2 * I)
-        self._product(h2, H, w.wgu, w.wgu_t, gu, N, 2 * I, H)
+        self._product(h2, H, w.wgu, w.wgu_t, gu, N, 2 * I, H, chain=chain)
         if not keep_norm:
             h2 = None
         act = self._empty(N, I)
         call("alodlm_swiglu_fwd", ptr(gu), ptr(act), N, I, c, st)
         y = self._empty(N, H)
-        self._product(act, I, w.wd, w.wd_t, y, N, H, I, epi=EPI_RESIDUAL, R=x1, ldr=H)
+        self._product(act, I, w.wd, w.wd_t, y, N, H, I, epi=EPI_RESIDUAL, R=x1, ldr=H, chain=chain)
         if save is not None:
             save.append((tag, x, rstd1, qkv, o, lse, x1, rstd2, gu, q, k, h1, h2))
         return y
 
-    def layer_bwd(self, dy, saved, w, gw, mask, rope, first=False, defer=None):
+    def layer_bwd(self, dy, saved, w, gw, mask, rope, first=False, defer=None, chain=False):
         """Backward of ``layer_fwd`` from its saved tuple: returns dx and adds
         the weight gradients into the float32 views ``gw`` (``first``: the four
         projection matrices' gradients are written instead of added; the norm
         weights' are always added).  With a list ``defer`` the four projection
         products are not run: their operands (A, lda, B, ldb, C, ldc, M, N;
         k = the rows) are appended to it in the order down, gate/up, O, QKV,
-        and the tensors stay alive through the list."""
+        and the tensors stay alive through the list.  ``chain``: as in
+        ``layer_fwd``."""
         _, x, rstd1, qkv, o, lse, x1, rstd2, gu, q, k, h1, h2 = saved
         d, N, st, c = self.dims, x.shape[0], self._stream(), self.code
         wepi = EPI_STORE if gw.stored else EPI_STORE_F32 if first else EPI_ACCUM
@@ -462,7 +465,7 @@ class Kernels:
         QD = d.heads * d.head_dim
         # ---- MLP: y = x1 + act . Wd^T  (the SwiGLU backward also rewrites act)
         dact = self._empty(N, I)
-        self._gemm(dy, H, 1, w.wd, I, 0, dact, I, N, I, H)
+        self._gemm(dy, H, 1, w.wd, I, 0, dact, I, N, I, H, chain=chain)
         act = self._empty(N, I)
         dgu = self._empty(N, 2 * I)
         call("alodlm_swiglu_bwd", ptr(dact), ptr(gu), ptr(dgu), ptr(act), N, I, c, st)
@@ -473,7 +476,7 @@ class Kernels:
             h2 = self._empty(N, H)
             call("alodlm_rmsnorm_fwd", ptr(x1), ptr(w.ln2), ptr(h2), None, N, H, d.eps, c, st)
         dh2 = self._empty(N, H)
-        self._gemm(dgu, 2 * I, 1, w.wgu, H, 0, dh2, H, N, H, 2 * I)
+        self._gemm(dgu, 2 * I, 1, w.wgu, H, 0, dh2, H, N, H, 2 * I, chain=chain)
         dw(dgu, 2 * I, h2, H, gw.wgu, H, 2 * I, H)
         del dgu, h2
         dx1 = self._empty(N, H)
@@ -483,7 +486,7 @@ class Kernels:
         del dh2
         # ---- attention: x1 = x + o . Wo^T
         do = self._empty(N, QD)
-        self._gemm(dx1, H, 1, w.wo, QD, 0, do, QD, N, QD, H)
+        self._gemm(dx1, H, 1, w.wo, QD, 0, do, QD, N, QD, H, chain=chain)
         dw(dx1, H, o, QD, gw.wo, QD, H, QD)
         if q is None:
             q = self._empty(N, QD)
@@ -502,7 +505,7 @@ class Kernels:
             h1 = self._empty(N, H)
             call("alodlm_rmsnorm_fwd", ptr(x), ptr(w.ln1), ptr(h1), None, N, H, d.eps, c, st)
         dh1 = self._empty(N, H)
-        self._gemm(dqkv, W, 1, w.wqkv, H, 0, dh1, H, N, H, W)
+        self._gemm(dqkv, W, 1, w.wqkv, H, 0, dh1, H, N, H, W, chain=chain)
         dw(dqkv, W, h1, H, gw.wqkv, H, W, H)
         del dqkv, h1
         dx = self._empty(N, H)

@@ -173,7 +173,8 @@ def device_info():
             "peak_bf16_tflops_from_clock": round(cus.value * 4096 * khz.value * 1e3 / 1e12, 1)}
 
 
-def gemm_bytes(A, lda, a_k, B, ldb, b_k, C, ldc, M, N, K, alpha=1.0, epi=0, R=None, ldr=0):
+def gemm_bytes(A, lda, a_k, B, ldb, b_k, C, ldc, M, N, K, alpha=1.0, epi=0, R=None, ldr=0,
+               chain=False):
     """Algorithmic HBM bytes of one GEMM launch: A and B read once (bf16), C
     written once (bf16 store, or float32 for the first contribution to a
     gradient), plus R read (residual) or the float32 C read and written back

@@ -337,6 +337,13 @@ int alodlm_attention_fwd(const void* q, const void* k, const void* v, int64_t ld
                          const int32_t* tiles, int64_t n_tiles, void* o, float* lse,
                          int64_t rows, int64_t nq, int64_t nkv, int64_t dh, int64_t block_size,
                          int dtype, void* stream);
+/* alodlm_attention_fwd with a row's sums in one order over its keys whatever the
+ * number of rows (bf16; alodlm_gemm_chain's counterpart). */
+int alodlm_attention_fwd_chain(const void* q, const void* k, const void* v, int64_t ldv,
+                               const int64_t* bounds, const int32_t* row_segment,
+                               const int32_t* tiles, int64_t n_tiles, void* o, float* lse,
+                               int64_t rows, int64_t nq, int64_t nkv, int64_t dh,
+                               int64_t block_size, int dtype, void* stream);
 int64_t alodlm_attention_ds_blocks(const int64_t* token_offsets, int64_t segments,
                                    int64_t block_size, int64_t* base_out);
 int64_t alodlm_attention_bwd_workspace(int64_t rows, int64_t nq, int64_t nkv, int64_t dh,

@@ -1,10 +1,12 @@
-"""ALoDLM.rollout in bf16: a row's sums run in one order whatever the other rows
-of the pack, and every output against 64 bits.
+"""ALoDLM.rollout and the fused step in bf16: a row's sums run in one order
+whatever the other rows of the pack, and every output of a rollout against 64
+bits.
 
-A rollout applies its layers once per depth to their own outputs, so a product
-summed in another order reaches every later depth; the word-embedding gradient,
-whose few nonzero rows dilute the table's root mean square, shows it at single
-elements by more than that root mean square."""
+Both apply their layers once per depth to their own outputs, so a product summed
+in another order reaches every later depth; the word-embedding gradient, whose
+few nonzero rows dilute the table's root mean square, shows it at single
+elements by more than that root mean square, and the step's loss, a difference
+of credits, by some percent."""
 
 import pytest
 import torch
@@ -100,6 +102,36 @@ def test_rollout_rows_do_not_depend_on_the_pack(length):
     for a, b in zip(alone[0] + alone[1], packed[0] + packed[1]):
         assert torch.equal(a, b[:n])
     assert torch.equal(alone[2], packed[2][:n])
+
+
+def _step(model, segments):
+    ids = torch.cat([s[0] for s in segments])
+    bounds = [0]
+    for s in segments:
+        bounds.append(bounds[-1] + len(s[0]))
+    draws = tuple(sum((s[1][i] for s in segments), []) for i in range(3))
+    u = [torch.cat(t).to(DEV) for t in zip(*(s[2] for s in segments))]
+    with torch.no_grad():
+        return model.engine().forward(ids.to(DEV), ids.to(DEV), torch.tensor(bounds), False,
+                                      exit_uniforms=u, draws=draws)[1]
+
+
+@pytest.mark.parametrize("length", [5, 20, 40, 130])
+def test_step_rows_do_not_depend_on_the_pack(length):
+    """The fused step's gates, exits and per-row cross-entropies of a segment are
+    bit-identical alone and beside other segments, and its gates and exits are
+    the rollout's."""
+    log(f"step of {length} tokens alone and in a pack")
+    model = cases._model("1.7b", 1, 512, 511, BF16, cases._generator(length))
+    segments = [_segment(model, n, n) for n in (length, 200, 15)]
+    alone, packed = _step(model, segments[:1]), _step(model, segments)
+    n = 2 * length
+    for name in ("gates", "ce", "entropy"):
+        assert torch.equal(alone[name], packed[name][:, :n]), name
+    assert torch.equal(alone["exits"], packed["exits"][:n])
+    _, gates, exits = _rollout(model, segments)
+    assert torch.equal(torch.stack(gates), packed["gates"].to(BF16))
+    assert torch.equal(exits, packed["exits"].long())
 
 
 @pytest.mark.parametrize("length", [3, 20, 130])
