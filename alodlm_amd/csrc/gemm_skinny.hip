@@ -255,7 +255,8 @@ void launch(const T* A, int64_t lda, const T* W, int64_t ldw, T* C, int64_t ldc,
 // of such workgroups or in many (12288 x 2048: 12.1 us against 16.8; float 21.1
 // against 25.4; 151936 x 2048: 129 against 142; but 24576 x 4096, one and a half
 // rounds: 45 against 40).  Two blocks and more want 16 weight rows everywhere (27
-// rows, 24576 x 4096: 51 us against 57).
+// rows, 24576 x 4096: 51 us against 57).  Timed over eight copies of the weight in
+// turn: the smaller shapes' copies stay in the 256 MB last-level cache.
 template <typename T>
 void launch_typed(const T* A, int64_t lda, const T* W, int64_t ldw, T* C, int64_t ldc, const T* R,
                   int64_t ldr, int M, int N, int K, float alpha, int epi, hipStream_t st) {
